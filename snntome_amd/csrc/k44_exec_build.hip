@@ -23,6 +23,8 @@ void K44GpuExecutorState::free_all() {
     aux_cmd.clear();
     ids.reset();
     stage.reset();
+    in_stage.reset();
+    ring.reset();
     history.reset();
     step_ctr.reset();
     id_tokens = hist_steps = 0;

@@ -234,34 +234,67 @@ void K44GpuExecutorState::set_history(uint32_t steps) {
     if (prog_active) build_program();  // the history pointer is in its argmax stage
 }
 
-void K44GpuExecutorState::upload_input_f32(const float *in, size_t n) {
-    const K44ResDesc &L = layout(plan_meta.input_res_key);
-    // whole planes (zero halos): the region may hold another tensor's data from the last run
-    std::vector<uint16_t> pad((size_t)plan_meta.input_c * L.channel_stride, 0u);
-    for (uint32_t ch = 0; ch < plan_meta.input_c; ++ch)
-        for (uint32_t y = 0; y < plan_meta.input_h; ++y)
-            for (uint32_t x = 0; x < plan_meta.input_w; ++x) {
-                const size_t src = ((size_t)ch * plan_meta.input_h + y) * plan_meta.input_w + x;
-                if (src < n) pad[L.canvas_offset(ch, y, x)] = float_to_half(in[src]);
-            }
-    K44_HIP(hipMemcpyAsync(canvas.p + plan_meta.input_off, pad.data(), pad.size() * 2u,
-                           hipMemcpyHostToDevice, stream));
-    K44_HIP(hipStreamSynchronize(stream));
+static k44dev::FrameLayout frame_layout(const K44ResDesc &L, uint32_t H, uint32_t W) {
+    k44dev::FrameLayout f{};
+    f.channel_stride = L.channel_stride;
+    f.H = H;
+    f.W = W;
+    f.x_step = 1u;
+    if (!L.is_1d_tokens) {
+        f.y0 = 1u;
+        f.x0 = L.is_image_token64 ? 1u : 4u;
+        f.x_step = L.is_image_token64 ? 64u : 1u;
+        f.row_stride = L.W_pad * f.x_step;
+    }
+    return f;
 }
 
-std::vector<float> K44GpuExecutorState::download_output_f32() {
-    const K44ResDesc &L = layout(plan_meta.output_res_key);
-    std::vector<uint16_t> pad((size_t)plan_meta.output_c * L.channel_stride);
-    K44_HIP(hipMemcpyAsync(pad.data(), canvas.p + plan_meta.output_off, pad.size() * 2u,
-                           hipMemcpyDeviceToHost, stream));
-    K44_HIP(hipStreamSynchronize(stream));
-    std::vector<float> out((size_t)plan_meta.output_c * plan_meta.output_h * plan_meta.output_w);
-    for (uint32_t ch = 0; ch < plan_meta.output_c; ++ch)
-        for (uint32_t y = 0; y < plan_meta.output_h; ++y)
-            for (uint32_t x = 0; x < plan_meta.output_w; ++x)
-                out[((size_t)ch * plan_meta.output_h + y) * plan_meta.output_w + x] =
-                    half_to_float(pad[L.canvas_offset(ch, y, x)]);
-    return out;
+// Input channels cross to the device as they are (at most kInStage bytes or one channel at a
+// time, in stream order) and are converted there.  Whole channels are written: the region may
+// hold another tensor's data from the last run.
+void K44GpuExecutorState::upload_input_f32(const float *in, size_t n) {
+    constexpr size_t kInStage = 16u << 20;
+    const k44dev::FrameLayout f = frame_layout(layout(plan_meta.input_res_key),
+                                                plan_meta.input_h, plan_meta.input_w);
+    const size_t per = (size_t)f.H * f.W;
+    const uint32_t C = plan_meta.input_c;
+    n = std::min(n, per * C);
+    const uint32_t step = (uint32_t)std::min<size_t>(C, std::max<size_t>(1u, kInStage / (per * 4u)));
+    if (in_stage.n < per * step) in_stage.alloc(per * step);
+    uint16_t *region = reinterpret_cast<uint16_t *>(canvas.p + plan_meta.input_off);
+    for (uint32_t c = 0; c < C; c += step) {
+        const uint32_t nc = std::min(step, C - c);
+        const size_t first = per * c;
+        const size_t cnt = first < n ? std::min(n - first, per * nc) : 0u;
+        if (cnt)
+            K44_HIP(hipMemcpyAsync(in_stage.p, in + first, cnt * 4u, hipMemcpyHostToDevice, stream));
+        K44_HIP(k44dev::launch_import_f32(region + (size_t)c * f.channel_stride, in_stage.p, cnt,
+                                          nc, f, stream));
+    }
+}
+
+// Output elements [0, n) converted on the device into the page-locked ring, chunk by chunk, and
+// copied out from there; returns when `out` holds them.
+void K44GpuExecutorState::download_output_f32(float *out, size_t n) {
+    const k44dev::FrameLayout f = frame_layout(layout(plan_meta.output_res_key),
+                                                plan_meta.output_h, plan_meta.output_w);
+    const uint16_t *region = reinterpret_cast<const uint16_t *>(canvas.p + plan_meta.output_off);
+    ring.need();
+    constexpr size_t kElems = HostRing::kChunk / 4u;
+    const size_t chunks = (n + kElems - 1u) / kElems;
+    auto take = [&](size_t i) {
+        K44_HIP(hipEventSynchronize(ring.ev[i & 1u]));
+        std::memcpy(out + i * kElems, ring.p + (i & 1u) * HostRing::kChunk,
+                    std::min(kElems, n - i * kElems) * 4u);
+    };
+    for (size_t i = 0; i < chunks; ++i) {
+        if (i >= 2u) take(i - 2u);
+        K44_HIP(k44dev::launch_export_f32(
+            reinterpret_cast<float *>(ring.p + (i & 1u) * HostRing::kChunk), region, i * kElems,
+            std::min(kElems, n - i * kElems), f, stream));
+        K44_HIP(hipEventRecord(ring.ev[i & 1u], stream));
+    }
+    for (size_t i = chunks > 2u ? chunks - 2u : 0u; i < chunks; ++i) take(i);
 }
 
 int K44GpuExecutorState::infer_f32(const float *in, int in_elems, float *out, int out_elems, float *ms_out) {
@@ -270,12 +303,13 @@ int K44GpuExecutorState::infer_f32(const float *in, int in_elems, float *out, in
     K44_HIP(hipEventRecord(ev0, stream));
     execute_plan();
     K44_HIP(hipEventRecord(ev1, stream));
-    K44_HIP(hipEventSynchronize(ev1));
+    download_output_f32(out, std::min((size_t)std::max(0, out_elems),
+                                      (size_t)plan_meta.output_c * plan_meta.output_h *
+                                          plan_meta.output_w));
+    K44_HIP(hipStreamSynchronize(stream));
     float ms = 0.0f;
     K44_HIP(hipEventElapsedTime(&ms, ev0, ev1));
     if (ms_out) *ms_out = ms;
-    const std::vector<float> y = download_output_f32();
-    std::memcpy(out, y.data(), std::min((size_t)std::max(0, out_elems), y.size()) * 4u);
     return 0;
 }
 

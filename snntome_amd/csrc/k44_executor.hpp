@@ -28,6 +28,7 @@
 #include "k44_tuning.hpp"
 #include "k44_wave_compiler.hpp"
 #include "k44wavec.h"
+#include "kernels/k44_hostio.hpp"
 #include "kernels/k44_launch.hpp"
 #include "kernels/k44_program.hpp"
 #include "kernels/k44_spatial.hpp"
@@ -66,6 +67,32 @@ struct DevBuf {
     void upload(const std::vector<T> &h) {
         alloc(h.size());
         if (!h.empty()) K44_HIP(hipMemcpy(p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+    }
+};
+
+// Page-locked transfer buffer of an executor (made at its first use): two chunks, so that the
+// host copies one out while a kernel fills the other.
+struct HostRing {
+    static constexpr size_t kChunk = 1u << 20;
+    char *p = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    HostRing() = default;
+    HostRing(const HostRing &) = delete;
+    HostRing &operator=(const HostRing &) = delete;
+    ~HostRing() { reset(); }
+    void reset() {
+        for (auto &e : ev) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+    }
+    void need() {
+        if (p) return;
+        for (auto &e : ev)
+            if (!e) K44_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        K44_HIP(hipHostMalloc((void **)&p, 2u * kChunk, hipHostMallocDefault));
     }
 };
 
@@ -270,6 +297,8 @@ struct K44GpuExecutorState {
     DevBuf<__half> canvas;
     DevBuf<uint32_t> ids, history, step_ctr;  // token ids (EMBED / ARGMAX), greedy history
     DevBuf<uint16_t> stage;  // packed strided canvas reads (wavec_gpu_read_canvas_2d)
+    DevBuf<float> in_stage;  // fp32 input channels on their way to the canvas (infer_f32)
+    HostRing ring;           // outputs on their way to pageable host memory
     uint32_t id_tokens = 0, hist_steps = 0;
     // Scratch shared by the commands of the plan (they run in order on one stream): split-K
     // partials of MFMA waves, per-chunk (value, index) partials of ARGMAX.
@@ -396,7 +425,7 @@ struct K44GpuExecutorState {
     void execute_plan();
     void set_history(uint32_t steps);
     void upload_input_f32(const float *in, size_t n);
-    std::vector<float> download_output_f32();
+    void download_output_f32(float *out, size_t n);
     int infer_f32(const float *in, int in_elems, float *out, int out_elems, float *ms_out);
 };
 

@@ -1,0 +1,117 @@
+"""infer_f32's device conversions: the canvas region it writes and the floats it returns, bit for
+bit against the host rounding rules, on every layout and at the values where rounding can go
+wrong (ties, subnormals, overflow, NaN payloads)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import cnn_oracle as co
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _floats(rng, n):
+    """Random floats, with every kind of special value among them."""
+    x = rng.standard_normal(n).astype(np.float32) * np.float32(10.0) ** rng.integers(-9, 6, n)
+    bits = np.array([0x00000000, 0x80000000, 0x7f800000, 0xff800000, 0x7f800001, 0x7fc00000,
+                     0xffffe000, 0x7f802000, 0x33000000, 0x33000001, 0x32ffffff, 0x387fe000,
+                     0x387ff000, 0x38801000, 0x477fefff, 0x477ff000, 0x3f801000, 0x3f803000,
+                     0x00000001, 0xb3800000], np.uint32).view(np.float32)
+    x = x.astype(np.float32)
+    k = min(n, bits.size)
+    x[rng.permutation(n)[:k]] = bits[:k]
+    return x
+
+
+def _half_bits(x):
+    """The oracle's rounding (its scalar form for the NaNs, whose payload numpy treats its own way)."""
+    x = np.ascontiguousarray(x, np.float32)
+    with np.errstate(over="ignore"):
+        h = x.astype(np.float16).view(np.uint16)
+    for i in np.flatnonzero(np.isnan(x)):
+        h[i] = orc.f32bits_to_f16(int(x.view(np.uint32)[i]))
+    return h
+
+
+def _widened(h):
+    """fp32 bits of fp16 bits (exact; NaN payloads shifted, not quieted)."""
+    h = np.ascontiguousarray(h, np.uint16)
+    f = h.view(np.float16).astype(np.float32).view(np.uint32)
+    nan = (h & 0x7c00) == 0x7c00
+    f[nan] = ((h[nan].astype(np.uint32) & 0x8000) << 16) | 0x7f800000 | \
+        ((h[nan].astype(np.uint32) & 0x3ff) << 13)
+    return f
+
+
+@pytest.mark.parametrize("C,W,extra", [(5, 1, 0), (3, 200, 0), (70000, 3, 0), (4, 64, 37)])
+def test_token_rows(wavec, C, W, extra):
+    """1-D inputs (ragged rows, more channels than a grid dimension holds, a short input)."""
+    rng = np.random.default_rng(C + W)
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", C, 1, W, is_1d=True)
+    g.add_swiglu("m", "x", "x", "y")
+    g.set_output("y")
+    plan = g.compile()
+    plan.init_gpu()
+    stride = (W + 63) // 64 * 64
+    plan.write_canvas(0, np.full(C * stride, 7.0, np.float16))  # stale data of an earlier run
+    n = C * W - extra
+    x = _floats(rng, n)
+    y = np.full((C, 1, W), -1.0, np.float32)
+    ms = ctypes.c_float(0)
+    fp = ctypes.POINTER(ctypes.c_float)
+    assert plan._lib.wavec_gpu_infer_f32(plan._handle, x.ctypes.data_as(fp), n,
+                                         y.ctypes.data_as(fp), y.size - extra,
+                                         ctypes.byref(ms)) == 0
+    full = np.zeros(C * W, np.float32)
+    full[:n] = x
+    want = np.zeros((C, stride), np.uint16)
+    want[:, :W] = _half_bits(full).reshape(C, W)
+    assert np.array_equal(plan.read_canvas(0, C * stride).reshape(C, stride), want)
+    off = int(plan.cmds[-1]["y_off"])
+    out = plan.read_canvas(off, C * stride).reshape(C, stride)[:, :W].reshape(-1)
+    ref = _widened(out)
+    got = y.reshape(-1)
+    assert np.array_equal(got[:n].view(np.uint32), ref[:n])
+    assert np.all(got[n:] == -1.0)  # elements past out_elems are not touched
+
+
+@pytest.mark.parametrize("H,W,frames", [(6, 64, 1), (7, 20, 1), (5, 30, 3), (4, 6, 64), (600, 700, 1)])
+def test_image_planes(wavec, H, W, frames):
+    """Padded planes (aligned and masked widths, several frames, 64 interleaved frames) and an
+    output of several transfer chunks."""
+    rng = np.random.default_rng(H * W)
+    C = 3
+    g = wavec.WaveGraph(kv_cache_max_seq=0, batch_size=frames)
+    g.add_input("img", C, H, W)
+    g.add_maxpool("p", "img", "y", kernel_size=5, stride=1, pad=2)
+    g.set_output("y")
+    plan = g.compile()
+    plan.init_gpu()
+    lay = co.Layout2D(H, W, frames, tok64=frames >= 64)
+    src = int(plan.cmds[0]["src_off"])
+    plan.write_canvas(src, np.full(C * lay.channel_stride, 3.0, np.float16))
+    x = _floats(rng, C * H * W).reshape(C, H, W)
+    x[np.isnan(x)] = 0.5  # (the pool's treatment of NaN is not what is tested here)
+    y, _ = plan.infer_f32(x)
+    want = np.zeros(C * lay.channel_stride, np.uint16)
+    want[lay.offsets(C)[0].ravel()] = _half_bits(x.ravel())
+    assert np.array_equal(plan.read_canvas(src, want.size), want)
+    out = plan.read_canvas(int(plan.cmds[-1]["y_off"]), C * lay.channel_stride)
+    ref = _widened(out[lay.offsets(C)[0].ravel()])
+    got = np.ascontiguousarray(y.reshape(frames, C, H, W)[0]).reshape(-1)
+    assert np.array_equal(got.view(np.uint32), ref)
+
+
+def test_token_rows_with_height(wavec):
+    """A token input declared with several rows per channel keeps the last one given."""
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", 16, 3, 10, is_1d=True)
+    g.add_linear("l", "x", "y", 16, 16, np.eye(16, dtype=np.float32))
+    g.set_output("y")
+    plan = g.compile()
+    x = np.arange(16 * 3 * 10, dtype=np.float32).reshape(16, 3, 10)
+    y, _ = plan.infer_f32(x)
+    assert np.array_equal(y[:, 0], x[:, 2])
