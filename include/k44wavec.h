@@ -288,10 +288,11 @@ int wavec_gpu_read_canvas_2d(void *handle, unsigned long long elem_off, unsigned
  *   narrow group launches as 1-D grids (each workgroup's wave from the prefix sums) / as
  *   (workgroups x waves) grids where those launch at most 1.5x the work items (automatic);
  *   "embed_refresh" 0 | 1 a decode embedding never / also (automatic) refreshes the compact
- *   state copy of the first layer's folded token shift (0: that RMSNorm + shift runs alone).
+ *   state copy of the first layer's folded token shift (0: that RMSNorm + shift runs alone);
+ *   "rows" 0 | 1 | 4 | 8 no row-table MFMA kernel / that many waves per tile in it.
  * wavec_set_tuning returns -1 (with a message) for an unknown key or a value the key does not
  * honour: -1 is always accepted; "dma_stages" takes 2 | 4, "ksplit" 1 | 4, "xcd_order" 0..2,
- * "t64_ring" 0..2, "narrow_chunk" >= 16, "narrow_wgs" >= 1, "prog_spin_ms" >= 0, every
+ * "t64_ring" 0..2, "rows" 0 | 1 | 4 | 8, "narrow_chunk" >= 16, "narrow_wgs" >= 1, "prog_spin_ms" >= 0, every
  * other key 0 | 1.  wavec_get_tuning returns the
  * value or -2 for an unknown key. */
 int wavec_set_tuning(const char *key, int value);

@@ -243,6 +243,92 @@ void K44GpuExecutorState::configure_mfma(const K44ExecCmd &c, WaveExec &wx, cons
     wx.w.upload(wh);
 }
 
+// Row-table MFMA configuration of a wave whose clusters (a multiple of 16 neurons) share an
+// index row but whose segments do not make whole k-steps.  Against the VALU gathers, which read
+// every row once per neuron: 4,096 neurons in clusters of 64 with 512 scattered synapses over
+// 256 tokens 480 -> 6.1 us, clusters of 16 with 16 synapses over 16 tokens 7.7 -> 2.8 us, a 3x3
+// convolution over 3 channels of 640 x 640 225 -> 49 us.  Returns false (nothing changed) where
+// the kernel does not apply.
+// wraw: [Cout][c.B] weights in segment order; tx / ty: tile tables of 2-D waves, else empty.
+bool K44GpuExecutorState::configure_rows(const K44ExecCmd &c, WaveExec &wx,
+                                         const std::vector<uint16_t> &wraw,
+                                         const std::vector<uint64_t> &starts,
+                                         const std::vector<uint32_t> &tx,
+                                         const std::vector<uint32_t> &ty) {
+    const int force = tune(Tune::Rows);
+    const uint32_t cl = c.cluster_size;
+    if (tune(Tune::Path) == 0 || force == 0 || cl == 0u || cl % 16u != 0u) return false;
+    // Planes of under 32 tiles and fan-ins under two k-steps: both kernels are one short
+    // latency chain (1x1 over 8..16 channels of 20 x 20: 6.5 us on the VALU gathers, 7.6-7.8
+    // here; 3x3 over 3 channels 7.6 and 7.7), the gathers with the shorter epilogue.
+    if (!tx.empty() && tx.size() < 32u && c.B_raw < 64u) return false;
+    const uint64_t lo = *std::min_element(starts.begin(), starts.end());
+    const uint64_t hi = *std::max_element(starts.begin(), starts.end()) +
+                        (uint64_t)(wx.S - 1u) * wx.step;
+    const uint32_t tx_hi = tx.empty() ? wx.tokens : *std::max_element(tx.begin(), tx.end()) + 64u;
+    if (hi - lo + tx_hi + 64u > 0xffffffffull) return false;
+    const uint32_t ttiles = wx.tokens / 64u, blocks = cl / 16u;
+    wx.rk_nb = blocks % 4u == 0u ? 4u : blocks % 3u == 0u ? 3u : blocks % 2u == 0u ? 2u : 1u;
+    wx.rk_subs = blocks / wx.rk_nb;
+    wx.rk_B = c.B_raw;
+    wx.rk_ksteps = (c.B_raw + 31u) / 32u;
+    wx.rk_base = lo;
+    const uint64_t wgs = (uint64_t)wx.rows * wx.rk_subs * ttiles;  // tiles x 64 tokens
+    // Waves per tile: 8 (4 for short rows) until tiles alone give 6 waves per CU (64 tiles x 16
+    // token tiles: 20.8 us with 4, 23.3 with 1; twice the tokens at clusters of 128: 57 and 44).
+    wx.rk_kw = wgs >= 1536u ? 1u : wx.rk_ksteps >= 8u ? 8u : 4u;
+    if (force > 0) wx.rk_kw = (uint32_t)force;
+    if ((uint64_t)wx.rows * wx.rk_subs > 0x7fffffffull || ttiles > 65535u) return false;
+    // 16-byte gathers need every row and tile on the 16-byte grid, else shifted into place
+    bool al = wx.step % 8u == 0u;
+    for (uint64_t s0 : starts) al = al && s0 % 8u == 0u;
+    for (uint32_t v : tx) al = al && v % 8u == 0u;
+    wx.rk_mis = !al;
+    uint32_t vec = 8u;
+    auto fit = [&](uint64_t v) {
+        while (vec > 1u && v % vec != 0u) vec = vec == 8u ? 4u : 1u;
+    };
+    fit(wx.y_off);
+    fit(wx.out_stride);
+    if (wx.has_res) fit(wx.res_off);
+    for (uint32_t v : ty) fit(v);
+    wx.rk_vec = wx.masked ? 1u : vec;
+    const size_t per = (size_t)wx.rk_ksteps * 32u;
+    std::vector<uint32_t> ro((size_t)wx.rows * per);
+    for (size_t r = 0; r < wx.rows; ++r)
+        for (size_t p = 0; p < per; ++p) {
+            const size_t q = std::min<size_t>(p, c.B_raw - 1u);  // past the row: zeroed in LDS
+            ro[r * per + p] = (uint32_t)(starts[r * wx.K + q / wx.S] + (q % wx.S) * wx.step - lo);
+        }
+    wx.roff.upload(ro);
+    // A fragments: [index row][sub-tile][k-step][16-neuron block][lane][8], zero past the row
+    std::vector<uint16_t> wf((size_t)c.Cout * per, 0u);
+    size_t dst = 0;
+    for (size_t t = 0; t < (size_t)wx.rows * wx.rk_subs; ++t)
+        for (uint32_t ks = 0; ks < wx.rk_ksteps; ++ks)
+            for (uint32_t b = 0; b < wx.rk_nb; ++b)
+                for (uint32_t l = 0; l < 64u; ++l, dst += 8u) {
+                    const size_t j = (t * wx.rk_nb + b) * 16u + (l & 15u);
+                    const uint32_t p0 = 32u * ks + 8u * (l >> 4);
+                    if (p0 >= c.B_raw) continue;
+                    std::memcpy(&wf[dst], &wraw[j * c.B + p0],
+                                std::min(8u, c.B_raw - p0) * 2u);
+                }
+    std::vector<__half> wh(wf.size());
+    std::memcpy(wh.data(), wf.data(), wf.size() * 2u);
+    wx.w.upload(wh);
+    wx.rowsk = true;
+    wx.path = "mfma_rows";
+    wx.why = "clusters of " + std::to_string(cl) + " share index rows of " +
+             std::to_string(c.B_raw) + " positions: row-table MFMA, " +
+             std::to_string(wx.rk_kw) + " waves per tile of " +
+             std::to_string(16u * wx.rk_nb) + " neurons x 64 tokens";
+    if (wx.rk_mis) wx.why += ", rows shifted into place";
+    if (wx.phase_order) wx.why += "; synapses regrouped by token phase";
+    wx.ksplit = wx.rk_kw;
+    return true;
+}
+
 void K44GpuExecutorState::build_wave(const K44ExecCmd &c, WaveExec &wx) {
     const auto &Lo = plan_meta.res_map.at(c.res_key_out);
     auto itin = plan_meta.res_map.find(c.res_key_in);
@@ -434,6 +520,8 @@ void K44GpuExecutorState::build_wave(const K44ExecCmd &c, WaveExec &wx) {
                                  "no dense MFMA tiling (cluster/segment/alignment)");
     if (wx.mfma) {
         configure_mfma(c, wx, wraw, rows, Lo.W);
+    } else if (configure_rows(c, wx, wraw, starts, {}, {})) {
+        // (kernel, row table and weights set there)
     } else {
         wx.path = "valu_gather_dot";
         wx.why = !nt_ok ? "neurons do not share index rows in tiles of 16..128 (cluster " +
@@ -667,7 +755,10 @@ void K44GpuExecutorState::build_wave2d(const K44ExecCmd &c, WaveExec &wx, const 
                                   (wx.masked ? ", halo columns not stored" : "");
         }
     }
-    if (!wx.mfma) wx.w.upload(wh);
+    // The others with clusters of >= 16 channels: row-table MFMA (64-frame interleaved images
+    // keep the VALU tile kernel).
+    if (!wx.mfma && !tok64) configure_rows(c, wx, wraw, starts, tx, ty);
+    if (!wx.mfma && !wx.rowsk) wx.w.upload(wh);
     wx.seg.upload(starts);
     std::vector<__half> bh(c.Cout);
     for (size_t j = 0; j < c.Cout; ++j) {

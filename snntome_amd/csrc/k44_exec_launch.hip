@@ -125,6 +125,35 @@ void K44GpuExecutorState::launch_wave(const WaveExec &w) {
             K44_HIP(k44dev::launch_halo_clear(canvas.p + w.y_off, w.cout, w.plane, stream));
         return;
     }
+    if (w.rowsk) {
+        k44dev::RowsArgs a{};
+        a.X = canvas.p + w.rk_base;
+        a.roff = w.roff.p;
+        a.Wf = w.w.p;
+        a.bias = w.bias.p;
+        a.cmap = w.cmap.p;
+        a.Y = canvas.p + w.y_off;
+        a.R = w.has_res ? canvas.p + w.res_off : nullptr;
+        a.tile_x = w.tile_x.p;
+        a.tile_y = w.tile_y.p;
+        a.out_stride = w.out_stride;
+        a.B = w.rk_B;
+        a.ksteps = w.rk_ksteps;
+        a.subs = w.rk_subs;
+        a.ttiles = w.tokens / 64u;
+        a.act = w.act;
+        a.vec = w.rk_vec;
+        if (w.tile2d && w.masked) {
+            a.mask_w = w.plane.W;
+            a.mask_h = w.plane.H;
+            a.mask_wpad = w.plane.W_pad;
+            a.mask_tpf = w.tiles_per_frame;
+        }
+        K44_HIP(k44dev::launch_mfma_rows(a, w.rows, w.rk_nb, w.rk_kw, w.rk_mis, stream));
+        if (w.tile2d)
+            K44_HIP(k44dev::launch_halo_clear(canvas.p + w.y_off, w.cout, w.plane, stream));
+        return;
+    }
     if (w.tile2d) {
         k44dev::GatherTileArgs a{};
         a.X = canvas.p;

@@ -30,6 +30,7 @@
 #include "k44wavec.h"
 #include "kernels/k44_hostio.hpp"
 #include "kernels/k44_launch.hpp"
+#include "kernels/k44_mfma_rows.hpp"
 #include "kernels/k44_program.hpp"
 #include "kernels/k44_spatial.hpp"
 
@@ -170,6 +171,12 @@ struct WaveExec {
     // the state range of a carried copy, counted as written when launches are grouped (so the
     // launch never joins one of the fold's readers)
     std::vector<std::pair<uint64_t, uint64_t>> carry_rng;
+    // Row-table MFMA kernel (k44_mfma_rows.hip): the positions of every index row as element
+    // offsets from rk_base, rk_kw waves per tile of 16 rk_nb neurons.
+    bool rowsk = false, rk_mis = false;
+    uint32_t rk_nb = 0, rk_kw = 0, rk_subs = 0, rk_ksteps = 0, rk_B = 0, rk_vec = 1;
+    uint64_t rk_base = 0;
+    DevBuf<uint32_t> roff;
     // 2-D spatial wave (VALU over the padded-plane tile layout): tile tables, output plane.
     bool tile2d = false;
     DevBuf<uint32_t> tile_x, tile_y;
@@ -373,6 +380,9 @@ struct K44GpuExecutorState {
     static bool streaming_gather(const WaveExec &wx);
     void configure_mfma(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
                         size_t rows, uint32_t width);
+    bool configure_rows(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
+                        const std::vector<uint64_t> &starts, const std::vector<uint32_t> &tx,
+                        const std::vector<uint32_t> &ty);
     void build_wave(const K44ExecCmd &c, WaveExec &wx);
     void build_wave2d(const K44ExecCmd &c, WaveExec &wx, const K44ResDesc &Lo,
                       const K44ResDesc &Li);

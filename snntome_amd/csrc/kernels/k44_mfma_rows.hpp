@@ -1,0 +1,30 @@
+// k44_mfma_rows.hpp — MFMA waves whose tiles gather arbitrary rows (see k44_mfma_rows.hip).
+#pragma once
+#include "k44_mfma_tile.hpp"
+
+namespace k44dev {
+
+struct RowsArgs {
+    const __half *X;       // canvas + the wave's lowest row offset
+    const uint32_t *roff;  // [index rows][32 ksteps] element offset of every position from X
+    const __half *Wf;      // A fragments [index row][sub-tile][k-step][NB][lane][8], zero padded
+    const __half *bias;    // [cout] or nullptr
+    const uint16_t *cmap;  // [cout] or nullptr
+    __half *Y;             // canvas + y_off
+    const __half *R;       // canvas + res_off or nullptr
+    const uint32_t *tile_x, *tile_y;  // per 64-token tile offsets (2-D waves); nullptr: 64 t
+    uint64_t out_stride;
+    uint32_t B, ksteps;    // positions per row, ceil(B / 32)
+    uint32_t subs;         // sub-tiles of 16 NB neurons per index row
+    uint32_t ttiles;       // 64-token tiles
+    int act;
+    uint32_t vec;          // output / residual rows: 8-, 4- or 1-element aligned stores
+    uint32_t mask_w, mask_h, mask_wpad, mask_tpf;  // as in MfmaTileArgs
+};
+
+// rows: index rows.  nb: 16-neuron blocks per workgroup (1..4); kw: waves that share a tile's
+// k-steps (1: four 64-token tiles per workgroup; 4 or 8: one).  mis: rows at any element offset.
+hipError_t launch_mfma_rows(const RowsArgs &a, uint32_t rows, uint32_t nb, uint32_t kw, bool mis,
+                            hipStream_t stream);
+
+}  // namespace k44dev
