@@ -22,7 +22,6 @@ void K44GpuExecutorState::free_all() {
     wave_cmd.clear();
     aux_cmd.clear();
     ids.reset();
-    stage.reset();
     in_stage.reset();
     ring.reset();
     history.reset();
@@ -964,6 +963,7 @@ void K44GpuExecutorState::init(const K44WavePlan &plan) {
     K44_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     K44_HIP(hipEventCreate(&ev0));
     K44_HIP(hipEventCreate(&ev1));
+    ring.need();  // (40 us: not at the first call)
     canvas.alloc((plan.canvas_elems + kCanvasSlack + 63u) / 64u * 64u + fold_elems);
     if (scratch_need) scratch.alloc(scratch_need);
     {

@@ -71,7 +71,7 @@ struct DevBuf {
     }
 };
 
-// Page-locked transfer buffer of an executor (made at its first use): two chunks, so that the
+// Page-locked transfer buffer of an executor, made with it: two chunks, so that the
 // host copies one out while a kernel fills the other.
 struct HostRing {
     static constexpr size_t kChunk = 1u << 20;
@@ -303,7 +303,6 @@ struct K44GpuExecutorState {
     std::vector<std::unique_ptr<MfmaGroupExec>> groups;
     DevBuf<__half> canvas;
     DevBuf<uint32_t> ids, history, step_ctr;  // token ids (EMBED / ARGMAX), greedy history
-    DevBuf<uint16_t> stage;  // packed strided canvas reads (wavec_gpu_read_canvas_2d)
     DevBuf<float> in_stage;  // fp32 input channels on their way to the canvas (infer_f32)
     HostRing ring;           // outputs on their way to pageable host memory
     uint32_t id_tokens = 0, hist_steps = 0;
@@ -436,6 +435,9 @@ struct K44GpuExecutorState {
     void set_history(uint32_t steps);
     void upload_input_f32(const float *in, size_t n);
     void download_output_f32(float *out, size_t n);
+    void read_rows(uint16_t *dst, uint64_t off, uint64_t rows, uint64_t row_stride, uint64_t cols);
+    template <typename Fill>
+    void to_host(void *dst, size_t bytes, Fill &&fill);
     int infer_f32(const float *in, int in_elems, float *out, int out_elems, float *ms_out);
 };
 

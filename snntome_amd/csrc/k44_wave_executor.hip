@@ -722,8 +722,7 @@ int wavec_gpu_read_canvas(void *h, unsigned long long off, unsigned long long n,
         if (!ex) throw std::runtime_error("wavec_gpu_init_plan has not succeeded for this handle");
         if (off > ex->plan_meta.canvas_elems || n > ex->plan_meta.canvas_elems - off)
             throw std::runtime_error("range outside the canvas");
-        K44_HIP(hipMemcpyAsync(dst, ex->canvas.p + off, n * 2u, hipMemcpyDeviceToHost, ex->stream));
-        K44_HIP(hipStreamSynchronize(ex->stream));
+        if (n) ex->read_rows(dst, off, 1u, n, n);
         return 0;
     });
 }
@@ -898,14 +897,7 @@ int wavec_gpu_read_canvas_2d(void *h, unsigned long long off, unsigned long long
         if (cols > row_stride || off > n || rows - 1u > (n - off) / row_stride ||
             off + (rows - 1u) * row_stride + cols > n)
             throw std::runtime_error("2-D range outside the canvas allocation");
-        // Packed on the device first (a staging buffer kept by the executor), then one copy.
-        if (ex->stage.n < rows * cols) ex->stage.alloc(rows * cols);
-        K44_HIP(k44dev::launch_gather_cols(ex->stage.p,
-                                           reinterpret_cast<const uint16_t *>(ex->canvas.p + off),
-                                           rows, row_stride, cols, ex->stream));
-        K44_HIP(hipMemcpyAsync(dst, ex->stage.p, rows * cols * 2u, hipMemcpyDeviceToHost,
-                               ex->stream));
-        K44_HIP(hipStreamSynchronize(ex->stream));
+        ex->read_rows(dst, off, rows, row_stride, cols);
         return 0;
     });
 }

@@ -3,8 +3,8 @@
 // Bound by the host link: 4 bytes per element over PCIe (about 55 GB/s on MI355X), against
 // about 5 us of device work per million elements.  The conversions replace a scalar host loop
 // over every element (1-2 ns per element and direction, on top of the same transfers): a dense
-// block over 200 tokens (205 k elements each way) 642 -> 281 us per call, an image block on a
-// 32 x 160 x 160 input (819 k in, 410 k out) 1952 -> 512 us.
+// block over 200 tokens (205 k elements each way) 642 -> 266 us per call, an image block on a
+// 32 x 160 x 160 input (819 k in, 410 k out) 1952 -> 472 us.
 #include "k44_hostio.hpp"
 
 #include <hip/hip_fp16.h>
@@ -143,6 +143,61 @@ hipError_t launch_export_f32(float *dst, const uint16_t *region, uint64_t first,
     hipLaunchKernelGGL(k44_export_f32_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, dst,
                        region, first, n, L,
                        reinterpret_cast<uintptr_t>(dst) % 16u == 0u ? 1u : 0u);
+    return hipGetLastError();
+}
+
+// Thread = 8 consecutive packed elements.  VEC: rows and both ends on the 16-byte grid.
+template <bool VEC, typename I>
+__global__ __launch_bounds__(256) void k44_pack_rows_kernel(uint16_t *dst, const uint16_t *src,
+                                                            I first, I n, uint64_t row_stride,
+                                                            I cols) {
+    for (I q = ((I)blockIdx.x * 256u + threadIdx.x) * 8u; q < n; q += (I)gridDim.x * 2048u) {
+        I r = (first + q) / cols, c = first + q - r * cols;
+        const uint16_t *p = src + (uint64_t)r * row_stride;
+        if constexpr (VEC) {
+            *reinterpret_cast<us8 *>(dst + q) = *reinterpret_cast<const us8 *>(p + c);
+        } else {
+            us8 v;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                v[i] = q + i < n ? p[c] : (unsigned short)0u;
+                if (++c == cols) {
+                    c = 0;
+                    p += q + i + 1u < n ? row_stride : 0u;
+                }
+            }
+            if (q + 8u <= n && reinterpret_cast<uintptr_t>(dst + q) % 16u == 0u) {
+                *reinterpret_cast<us8 *>(dst + q) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (q + i < n) dst[q + i] = v[i];
+            }
+        }
+    }
+}
+
+template <bool VEC>
+static void pack_rows(uint16_t *dst, const uint16_t *src, uint64_t first, uint64_t n,
+                      uint64_t row_stride, uint64_t cols, hipStream_t stream) {
+    const dim3 grid((uint32_t)std::min<uint64_t>((n + 2047u) / 2048u, 2048u));
+    if (first + n < (1ull << 31))  // (32-bit division; the loop's last step stays below 2^32)
+        hipLaunchKernelGGL((k44_pack_rows_kernel<VEC, uint32_t>), grid, dim3(256), 0, stream, dst,
+                           src, (uint32_t)first, (uint32_t)n, row_stride, (uint32_t)cols);
+    else
+        hipLaunchKernelGGL((k44_pack_rows_kernel<VEC, uint64_t>), grid, dim3(256), 0, stream, dst,
+                           src, first, n, row_stride, cols);
+}
+
+hipError_t launch_pack_rows(uint16_t *dst, const uint16_t *src, uint64_t first, uint64_t n,
+                            uint64_t row_stride, uint64_t cols, hipStream_t stream) {
+    if (n == 0u) return hipSuccess;
+    const bool vec = (first | n | row_stride | cols) % 8u == 0u &&
+                     (reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) % 16u == 0u;
+    if (vec)
+        pack_rows<true>(dst, src, first, n, row_stride, cols, stream);
+    else
+        pack_rows<false>(dst, src, first, n, row_stride, cols, stream);
     return hipGetLastError();
 }
 

@@ -24,4 +24,9 @@ hipError_t launch_import_f32(uint16_t *region, const float *in, uint64_t n_in, u
 hipError_t launch_export_f32(float *dst, const uint16_t *region, uint64_t first, uint64_t n,
                              const FrameLayout &L, hipStream_t stream);
 
+// dst[0 .. n) = elements [first, first + n) of [rows][cols], row r at src + r * row_stride,
+// packed.  dst may be page-locked host memory.
+hipError_t launch_pack_rows(uint16_t *dst, const uint16_t *src, uint64_t first, uint64_t n,
+                            uint64_t row_stride, uint64_t cols, hipStream_t stream);
+
 }  // namespace k44dev

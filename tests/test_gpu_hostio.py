@@ -115,3 +115,43 @@ def test_token_rows_with_height(wavec):
     x = np.arange(16 * 3 * 10, dtype=np.float32).reshape(16, 3, 10)
     y, _ = plan.infer_f32(x)
     assert np.array_equal(y[:, 0], x[:, 2])
+
+
+def _hip():
+    """The HIP runtime this process already uses."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    return ctypes.CDLL(path)
+
+
+@pytest.mark.parametrize("pinned,shift", [(False, 0), (True, 0), (True, 1)])
+@pytest.mark.parametrize("rows,stride,cols,off", [
+    (1, 5, 5, 0), (37, 64, 9, 3), (700, 128, 128, 8), (900, 1024, 1000, 64), (2000, 640, 577, 1)])
+def test_canvas_reads(wavec, pinned, shift, rows, stride, cols, off):
+    """read_canvas_2d into pageable memory (one and several transfer chunks) and into page-locked
+    memory written in place, aligned and not; nothing past the destination is touched."""
+    rng = np.random.default_rng(rows)
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", 2100, 1, 1024, is_1d=True)
+    g.add_swiglu("m", "x", "x", "y")
+    plan = g.compile()
+    plan.init_gpu()
+    data = rng.integers(0, 65536, off + rows * stride + 8, dtype=np.uint16)
+    plan.write_canvas(0, data)
+    want = np.lib.stride_tricks.as_strided(data[off:], (rows, cols), (2 * stride, 2)).reshape(-1)
+    if not pinned:
+        assert np.array_equal(plan.read_canvas_2d(off, rows, stride, cols).reshape(-1), want)
+        assert np.array_equal(plan.read_canvas(off, rows * stride), data[off:off + rows * stride])
+        return
+    hip, p = _hip(), ctypes.c_void_p()
+    n = rows * cols + 16
+    assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(2 * n), 0) == 0
+    buf = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_uint16)), (n,))
+    buf[:] = 0xabcd
+    try:
+        dst = ctypes.cast(p.value + 2 * shift, ctypes.POINTER(ctypes.c_uint16))
+        assert plan._lib.wavec_gpu_read_canvas_2d(plan._handle, off, rows, stride, cols, dst) == 0
+        assert np.array_equal(buf[shift:shift + rows * cols], want)
+        assert np.all(buf[:shift] == 0xabcd) and np.all(buf[shift + rows * cols:] == 0xabcd)
+    finally:
+        del buf
+        hip.hipHostFree(p)
