@@ -224,60 +224,53 @@ void K44GpuExecutorState::configure_mfma(const K44ExecCmd &c, WaveExec &wx, cons
         if (wx.kgroups > 1u) wx.part_floats = (size_t)wx.kgroups * c.Cout * wx.tokens;
     }
     wx.ksteps = c.B_raw / 32u;
-    const uint32_t nb = cl / 16u;
-    // A fragments: [tile][k-step][16-neuron block][lane][8]; lane l holds neuron
-    // 16*blk + (l & 15), positions 32*ks + 8*(l >> 4) .. +8 of the tile's index row.
-    std::vector<uint16_t> wf((size_t)c.Cout * c.B_raw);
-    for (size_t t = 0; t < rows; ++t)
-        for (uint32_t ks = 0; ks < wx.ksteps; ++ks)
-            for (uint32_t b = 0; b < nb; ++b)
-                for (uint32_t l = 0; l < 64u; ++l) {
-                    const size_t dst = (((t * wx.ksteps + ks) * nb + b) * 64u + l) * 8u;
-                    const size_t j = t * cl + 16u * b + (l & 15u);
-                    const size_t src = j * c.B + 32u * ks + 8u * (l >> 4);
-                    std::memcpy(&wf[dst], &wraw[src], 16);
-                }
-    std::vector<__half> wh(wf.size());
-    std::memcpy(wh.data(), wf.data(), wf.size() * 2u);
-    wx.w.upload(wh);
+    upload_fragments(c, wx, wraw, rows);
 }
 
-// Row-table MFMA configuration of a wave whose clusters (a multiple of 16 neurons) share an
-// index row but whose segments do not make whole k-steps.  Against the VALU gathers, which read
-// every row once per neuron: 4,096 neurons in clusters of 64 with 512 scattered synapses over
-// 256 tokens 480 -> 6.1 us, clusters of 16 with 16 synapses over 16 tokens 7.7 -> 2.8 us, a 3x3
-// convolution over 3 channels of 640 x 640 225 -> 49 us.  Returns false (nothing changed) where
-// the kernel does not apply.
-// wraw: [Cout][c.B] weights in segment order; tx / ty: tile tables of 2-D waves, else empty.
-bool K44GpuExecutorState::configure_rows(const K44ExecCmd &c, WaveExec &wx,
-                                         const std::vector<uint16_t> &wraw,
-                                         const std::vector<uint64_t> &starts,
-                                         const std::vector<uint32_t> &tx,
-                                         const std::vector<uint32_t> &ty) {
-    const int force = tune(Tune::Rows);
+// A fragments: [tile][k-step][16-neuron block][lane][8]; lane l holds neuron 16*blk + (l & 15),
+// positions 32*ks + 8*(l >> 4) .. +8 of the tile's index row (zeros past its end).
+void K44GpuExecutorState::upload_fragments(const K44ExecCmd &c, WaveExec &wx,
+                                           const std::vector<uint16_t> &wraw, size_t rows) {
+    const uint32_t cl = c.cluster_size, nb = cl / 16u, ksteps = (c.B_raw + 31u) / 32u;
+    const size_t n = (size_t)c.Cout * ksteps * 32u;
+    std::unique_ptr<uint16_t[]> wf(new uint16_t[n]);  // (every element written below)
+    uint16_t *dst = wf.get();
+    for (size_t t = 0; t < rows; ++t)
+        for (uint32_t ks = 0; ks < ksteps; ++ks)
+            for (uint32_t b = 0; b < nb; ++b)
+                for (uint32_t l = 0; l < 64u; ++l, dst += 8u) {
+                    const uint32_t p0 = 32u * ks + 8u * (l >> 4);
+                    const uint16_t *src = &wraw[(t * cl + 16u * b + (l & 15u)) * c.B + p0];
+                    if (p0 + 8u <= c.B_raw)
+                        std::memcpy(dst, src, 16);
+                    else
+                        for (uint32_t e = 0; e < 8u; ++e) dst[e] = p0 + e < c.B_raw ? src[e] : 0u;
+                }
+    wx.w.alloc(n);
+    K44_HIP(hipMemcpy(wx.w.p, wf.get(), n * 2u, hipMemcpyHostToDevice));
+}
+
+// Whether the row-table MFMA kernel can run a wave of clusters of a multiple of 16 neurons (any
+// positions, 32-bit offsets between them), and its shape and table if so.  tx / ty: tile tables
+// of 2-D waves, else empty.
+bool K44GpuExecutorState::rows_shape(const K44ExecCmd &c, WaveExec &wx,
+                                     const std::vector<uint64_t> &starts,
+                                     const std::vector<uint32_t> &tx,
+                                     const std::vector<uint32_t> &ty) {
     const uint32_t cl = c.cluster_size;
-    if (tune(Tune::Path) == 0 || force == 0 || cl == 0u || cl % 16u != 0u) return false;
-    // Planes of under 32 tiles and fan-ins under two k-steps: both kernels are one short
-    // latency chain (1x1 over 8..16 channels of 20 x 20: 6.5 us on the VALU gathers, 7.6-7.8
-    // here; 3x3 over 3 channels 7.6 and 7.7), the gathers with the shorter epilogue.
-    if (!tx.empty() && tx.size() < 32u && c.B_raw < 64u) return false;
+    if (tune(Tune::Path) == 0 || tune(Tune::Rows) == 0 || cl == 0u || cl % 16u != 0u) return false;
     const uint64_t lo = *std::min_element(starts.begin(), starts.end());
     const uint64_t hi = *std::max_element(starts.begin(), starts.end()) +
                         (uint64_t)(wx.S - 1u) * wx.step;
     const uint32_t tx_hi = tx.empty() ? wx.tokens : *std::max_element(tx.begin(), tx.end()) + 64u;
     if (hi - lo + tx_hi + 64u > 0xffffffffull) return false;
-    const uint32_t ttiles = wx.tokens / 64u, blocks = cl / 16u;
+    const uint32_t blocks = cl / 16u;
     wx.rk_nb = blocks % 4u == 0u ? 4u : blocks % 3u == 0u ? 3u : blocks % 2u == 0u ? 2u : 1u;
     wx.rk_subs = blocks / wx.rk_nb;
     wx.rk_B = c.B_raw;
     wx.rk_ksteps = (c.B_raw + 31u) / 32u;
     wx.rk_base = lo;
-    const uint64_t wgs = (uint64_t)wx.rows * wx.rk_subs * ttiles;  // tiles x 64 tokens
-    // Waves per tile: 8 (4 for short rows) until tiles alone give 6 waves per CU (64 tiles x 16
-    // token tiles: 20.8 us with 4, 23.3 with 1; twice the tokens at clusters of 128: 57 and 44).
-    wx.rk_kw = wgs >= 1536u ? 1u : wx.rk_ksteps >= 8u ? 8u : 4u;
-    if (force > 0) wx.rk_kw = (uint32_t)force;
-    if ((uint64_t)wx.rows * wx.rk_subs > 0x7fffffffull || ttiles > 65535u) return false;
+    if ((uint64_t)wx.rows * wx.rk_subs > 0xffffffull || wx.rk_ttiles() > 65535u) return false;
     // 16-byte gathers need every row and tile on the 16-byte grid, else shifted into place
     bool al = wx.step % 8u == 0u;
     for (uint64_t s0 : starts) al = al && s0 % 8u == 0u;
@@ -293,39 +286,34 @@ bool K44GpuExecutorState::configure_rows(const K44ExecCmd &c, WaveExec &wx,
     for (uint32_t v : ty) fit(v);
     wx.rk_vec = wx.masked ? 1u : vec;
     const size_t per = (size_t)wx.rk_ksteps * 32u;
-    std::vector<uint32_t> ro((size_t)wx.rows * per);
+    wx.roff_h.resize((size_t)wx.rows * per);
     for (size_t r = 0; r < wx.rows; ++r)
-        for (size_t p = 0; p < per; ++p) {
-            const size_t q = std::min<size_t>(p, c.B_raw - 1u);  // past the row: zeroed in LDS
-            ro[r * per + p] = (uint32_t)(starts[r * wx.K + q / wx.S] + (q % wx.S) * wx.step - lo);
-        }
-    wx.roff.upload(ro);
-    // A fragments: [index row][sub-tile][k-step][16-neuron block][lane][8], zero past the row
-    std::vector<uint16_t> wf((size_t)c.Cout * per, 0u);
-    size_t dst = 0;
-    for (size_t t = 0; t < (size_t)wx.rows * wx.rk_subs; ++t)
-        for (uint32_t ks = 0; ks < wx.rk_ksteps; ++ks)
-            for (uint32_t b = 0; b < wx.rk_nb; ++b)
-                for (uint32_t l = 0; l < 64u; ++l, dst += 8u) {
-                    const size_t j = (t * wx.rk_nb + b) * 16u + (l & 15u);
-                    const uint32_t p0 = 32u * ks + 8u * (l >> 4);
-                    if (p0 >= c.B_raw) continue;
-                    std::memcpy(&wf[dst], &wraw[j * c.B + p0],
-                                std::min(8u, c.B_raw - p0) * 2u);
-                }
-    std::vector<__half> wh(wf.size());
-    std::memcpy(wh.data(), wf.data(), wf.size() * 2u);
-    wx.w.upload(wh);
-    wx.rowsk = true;
-    wx.path = "mfma_rows";
-    wx.why = "clusters of " + std::to_string(cl) + " share index rows of " +
-             std::to_string(c.B_raw) + " positions: row-table MFMA, " +
-             std::to_string(wx.rk_kw) + " waves per tile of " +
-             std::to_string(16u * wx.rk_nb) + " neurons x 64 tokens";
-    if (wx.rk_mis) wx.why += ", rows shifted into place";
-    if (wx.phase_order) wx.why += "; synapses regrouped by token phase";
-    wx.ksplit = wx.rk_kw;
+        for (size_t k = 0; k < wx.K; ++k)
+            for (size_t q = 0; q < wx.S; ++q)
+                wx.roff_h[r * per + k * wx.S + q] = (uint32_t)(starts[r * wx.K + k] + q * wx.step - lo);
+    for (size_t r = 0; r < wx.rows; ++r)  // past the row: zeroed in LDS
+        std::fill(&wx.roff_h[r * per] + c.B_raw, &wx.roff_h[r * per] + per,
+                  wx.roff_h[r * per + c.B_raw - 1u]);
+    wx.rows_ok = true;
     return true;
+}
+
+// Waves per tile: 8 (4 for short rows), 4 once there are 512 tiles of 64 tokens (64 neuron tiles
+// of 8,192 inputs over 512 tokens, rows from HBM: 110 us with 8, 88 with 4; 64 x 8 tiles of 600
+// scattered inputs 11.1 and 10.7), 1 once the tiles alone give 6 waves per CU (64 x 16 tiles: 20.8
+// us with 4, 23.3 with 1; twice the tiles: 57 and 44).
+uint32_t K44GpuExecutorState::rows_waves(uint64_t tiles, uint32_t ksteps) {
+    if (tune(Tune::Rows) > 0) return (uint32_t)tune(Tune::Rows);
+    return tiles >= 1536u ? 1u : ksteps >= 8u && tiles < 512u ? 8u : 4u;
+}
+
+void K44GpuExecutorState::use_rows(WaveExec &wx, uint32_t kw) {
+    wx.rowsk = true;
+    wx.rk_kw = kw;
+    wx.roff.upload(wx.roff_h);
+    wx.why += "; row-table MFMA kernel, " + std::to_string(kw) + " waves per tile of " +
+              std::to_string(16u * wx.rk_nb) + " neurons x 64 tokens";
+    if (wx.rk_mis && !wx.mis) wx.why += ", rows shifted into place";
 }
 
 void K44GpuExecutorState::build_wave(const K44ExecCmd &c, WaveExec &wx) {
@@ -519,8 +507,21 @@ void K44GpuExecutorState::build_wave(const K44ExecCmd &c, WaveExec &wx) {
                                  "no dense MFMA tiling (cluster/segment/alignment)");
     if (wx.mfma) {
         configure_mfma(c, wx, wraw, rows, Lo.W);
-    } else if (configure_rows(c, wx, wraw, starts, {}, {})) {
-        // (kernel, row table and weights set there)
+        // (form_runs decides, launch by launch; switches that pick one of the other kernels keep it)
+        if (!wx.narrow && tune(Tune::Dma) < 0 && tune(Tune::DmaStages) < 0 &&
+            tune(Tune::DmaProd) < 0 && tune(Tune::SplitK) != 0)
+            rows_shape(c, wx, starts, {}, {});
+    } else if (rows_shape(c, wx, starts, {}, {})) {
+        // Against the VALU gathers, which read every row once per neuron: 4,096 neurons in
+        // clusters of 64 with 512 scattered synapses over 256 tokens 480 -> 6.1 us, clusters of
+        // 16 with 16 synapses over 16 tokens 7.7 -> 2.8 us.
+        wx.path = "mfma_rows";
+        wx.why = "clusters of " + std::to_string(cl) + " share index rows of " +
+                 std::to_string(c.B_raw) + " positions";
+        if (wx.phase_order) wx.why += "; synapses regrouped by token phase";
+        use_rows(wx, rows_waves(wx.rk_tiles(), wx.rk_ksteps));
+        wx.roff_h = {};
+        upload_fragments(c, wx, wraw, rows);
     } else {
         wx.path = "valu_gather_dot";
         wx.why = !nt_ok ? "neurons do not share index rows in tiles of 16..128 (cluster " +
@@ -742,7 +743,24 @@ void K44GpuExecutorState::build_wave2d(const K44ExecCmd &c, WaveExec &wx, const 
         for (uint64_t s0 : starts) al = al && s0 % 8u == 0u;
         for (uint32_t v : tx) al = al && v % 64u == 0u;
         for (uint32_t v : ty) al = al && v % 64u == 0u;
-        if (ok && (al || !tok64)) {
+        // Planes of under 32 tiles and fan-ins under two k-steps: gathers and row-table kernel
+        // are one short latency chain (1x1 over 8..16 channels of 20 x 20: 6.5 us on the
+        // gathers, 7.6-7.8; 3x3 over 3 channels 7.6 and 7.7), the gathers with the shorter
+        // epilogue.  64-frame images keep their kernels.
+        if (!tok64 && tune(Tune::Path) != 0 && (ok || wx.tiles >= 32u || c.B_raw >= 64u) &&
+            rows_shape(c, wx, starts, tx, ty)) {
+            // Against the VALU tile kernel, a 3x3 convolution over 3 channels of 640 x 640
+            // 225 -> 49 us; against the register-staged tile kernel (one wave per 64 tokens and
+            // no split), an image block on 64 channels of 256 x 256 402 -> 180 us.
+            wx.path = ok ? "mfma_tile" : "mfma_rows";
+            wx.why = "neurons share index rows in tiles of " + std::to_string(cl) +
+                     "; single-frame image: tile tables" +
+                     (wx.masked ? ", halo columns not stored" : "");
+            if (wx.phase_order) wx.why += "; synapses regrouped by token phase";
+            use_rows(wx, rows_waves(wx.rk_tiles(), wx.rk_ksteps));
+            wx.roff_h = {};
+            upload_fragments(c, wx, wraw, rows);
+        } else if (ok && (al || !tok64)) {
             wx.mfma = true;
             wx.mis = !al;
             wx.epi_scalar = !tok64;
@@ -754,9 +772,6 @@ void K44GpuExecutorState::build_wave2d(const K44ExecCmd &c, WaveExec &wx, const 
                                   (wx.masked ? ", halo columns not stored" : "");
         }
     }
-    // The others with clusters of >= 16 channels: row-table MFMA (64-frame interleaved images
-    // keep the VALU tile kernel).
-    if (!wx.mfma && !tok64) configure_rows(c, wx, wraw, starts, tx, ty);
     if (!wx.mfma && !wx.rowsk) wx.w.upload(wh);
     wx.seg.upload(starts);
     std::vector<__half> bh(c.Cout);
@@ -1147,7 +1162,7 @@ uint32_t K44GpuExecutorState::epi_workgroups(const WaveExec &w) {
 void K44GpuExecutorState::upload_mfma_descriptors() {
     for (auto &wp : waves) {
         WaveExec &w = *wp;
-        if (!w.mfma) continue;
+        if (!w.mfma || w.rowsk) continue;
         w.items = w.rows * (w.narrow ? 1u : w.tokens / w.mt) * w.kgroups;
         w.epi_items = epi_workgroups(w);
         const k44dev::MfmaTileArgs one = mfma_args(w, scratch.p, false);
@@ -1157,8 +1172,22 @@ void K44GpuExecutorState::upload_mfma_descriptors() {
     }
     for (auto &gp : groups) {
         MfmaGroupExec &g = *gp;
-        std::vector<k44dev::MfmaTileArgs> args;
         std::vector<uint32_t> start = {0u};
+        if (g.rowsk) {
+            std::vector<k44dev::RowsArgs> ra;
+            g.rk_ttiles = 0;
+            for (size_t m : g.members) {
+                const WaveExec &w = *waves[m];
+                ra.push_back(rows_args(w, true));
+                start.push_back(start.back() + w.rows * w.rk_subs);
+                g.rk_ttiles = std::max(g.rk_ttiles, w.rk_ttiles());
+            }
+            g.rk_cols = start.back();
+            g.rk_args.upload(ra);
+            g.start.upload(start);
+            continue;
+        }
+        std::vector<k44dev::MfmaTileArgs> args;
         uint32_t epi_max = 0, item_max = 0;
         size_t off = 0;
         // Device order of the members: with per-wave XCD shares, waves with the most stages

@@ -106,6 +106,42 @@ void K44GpuExecutorState::launch_mfma_group(const k44dev::MfmaGroup &d, uint32_t
     if (epi_items) K44_HIP(k44dev::launch_splitk_epilogue(d, epi_items, stream));
 }
 
+k44dev::RowsArgs K44GpuExecutorState::rows_args(const WaveExec &w, bool fused) const {
+    k44dev::RowsArgs a{};
+    a.X = canvas.p + w.rk_base;
+    a.roff = w.roff.p;
+    a.Wf = w.w.p;
+    a.bias = w.bias.p;
+    a.cmap = w.cmap.p;
+    a.Y = canvas.p + (fused ? w.y_off_run : w.y_off);
+    a.R = w.has_res ? canvas.p + w.res_off : nullptr;
+    a.tile_x = w.tile_x.p;
+    a.tile_y = w.tile_y.p;
+    a.out_stride = w.out_stride;
+    a.B = w.rk_B;
+    a.ksteps = w.rk_ksteps;
+    a.blocks = w.cluster / 16u;
+    a.subs = w.rk_subs;
+    a.ttiles = w.rk_ttiles();
+    a.act = w.act;
+    a.vec = w.rk_vec;
+    if (w.tile2d && w.masked) {
+        a.mask_w = w.plane.W;
+        a.mask_h = w.plane.H;
+        a.mask_wpad = w.plane.W_pad;
+        a.mask_tpf = w.tiles_per_frame;
+    }
+    return a;
+}
+
+// One wave alone, as compiled (a wave's output never moves past the canvas unless folded).
+void K44GpuExecutorState::launch_rows(const WaveExec &w) {
+    k44dev::RowsLaunch l;
+    l.one = rows_args(w, false);
+    K44_HIP(k44dev::launch_mfma_rows(l, w.rows * w.rk_subs, w.rk_ttiles(), w.rk_nb, w.rk_kw,
+                                     w.rk_mis, stream));
+}
+
 void K44GpuExecutorState::launch_mfma(const WaveExec &w) {
     const k44dev::MfmaGroup d{w.one_args.p, w.one_start.p, 1u, xcd_order};
     launch_mfma_group(d, w.cluster, w.mt, w.rows_per_stage, w.items, w.epi_items, w.dma,
@@ -113,43 +149,34 @@ void K44GpuExecutorState::launch_mfma(const WaveExec &w) {
 }
 
 void K44GpuExecutorState::launch_group(const MfmaGroupExec &g) {
+    if (g.rowsk) {
+        const WaveExec &w = *waves[g.members[0]];
+        k44dev::RowsLaunch l;
+        if (g.members.size() > 1u) {
+            l.waves = g.rk_args.p;
+            l.start = g.start.p;
+            l.n = (uint32_t)g.members.size();
+        } else {
+            l.one = rows_args(w, true);
+        }
+        K44_HIP(k44dev::launch_mfma_rows(l, g.rk_cols, g.rk_ttiles, w.rk_nb, w.rk_kw, w.rk_mis,
+                                         stream));
+        return;
+    }
     const k44dev::MfmaGroup d{g.args.p, g.start.p, (uint32_t)g.members.size(), xcd_order};
     launch_mfma_group(d, g.nt, g.mt, g.rows, g.items, g.epi_items, g.dma, g.dshape,
                       g.prod, g.max_items, g.mis, g.pre);
 }
 
 void K44GpuExecutorState::launch_wave(const WaveExec &w) {
-    if (w.mfma) {
-        launch_mfma(w);
+    if (w.rowsk) {
+        launch_rows(w);
         if (w.tile2d)
             K44_HIP(k44dev::launch_halo_clear(canvas.p + w.y_off, w.cout, w.plane, stream));
         return;
     }
-    if (w.rowsk) {
-        k44dev::RowsArgs a{};
-        a.X = canvas.p + w.rk_base;
-        a.roff = w.roff.p;
-        a.Wf = w.w.p;
-        a.bias = w.bias.p;
-        a.cmap = w.cmap.p;
-        a.Y = canvas.p + w.y_off;
-        a.R = w.has_res ? canvas.p + w.res_off : nullptr;
-        a.tile_x = w.tile_x.p;
-        a.tile_y = w.tile_y.p;
-        a.out_stride = w.out_stride;
-        a.B = w.rk_B;
-        a.ksteps = w.rk_ksteps;
-        a.subs = w.rk_subs;
-        a.ttiles = w.tokens / 64u;
-        a.act = w.act;
-        a.vec = w.rk_vec;
-        if (w.tile2d && w.masked) {
-            a.mask_w = w.plane.W;
-            a.mask_h = w.plane.H;
-            a.mask_wpad = w.plane.W_pad;
-            a.mask_tpf = w.tiles_per_frame;
-        }
-        K44_HIP(k44dev::launch_mfma_rows(a, w.rows, w.rk_nb, w.rk_kw, w.rk_mis, stream));
+    if (w.mfma) {
+        launch_mfma(w);
         if (w.tile2d)
             K44_HIP(k44dev::launch_halo_clear(canvas.p + w.y_off, w.cout, w.plane, stream));
         return;
@@ -341,6 +368,7 @@ void K44GpuExecutorState::to_host(void *dst, size_t bytes, Fill &&fill) {
         K44_HIP(hipStreamSynchronize(stream));
         return;
     }
+    std::lock_guard<std::recursive_mutex> lk(io);
     constexpr size_t kChunk = HostRing::kChunk;
     if (bytes <= kChunk) {
         fill(ring.p, 0u, bytes);
@@ -384,6 +412,7 @@ void K44GpuExecutorState::read_rows(uint16_t *dst, uint64_t off, uint64_t rows, 
 
 int K44GpuExecutorState::infer_f32(const float *in, int in_elems, float *out, int out_elems, float *ms_out) {
     if (!initialized) throw std::runtime_error("executor not initialised");
+    std::lock_guard<std::recursive_mutex> lk(io);  // (the ring holds a small input until it ran)
     upload_input_f32(in, (size_t)std::max(0, in_elems));
     K44_HIP(hipEventRecord(ev0, stream));
     execute_plan();

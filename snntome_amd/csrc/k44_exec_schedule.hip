@@ -1192,6 +1192,44 @@ void K44GpuExecutorState::form_runs() {
             }
         }
     }
+    // Row-table kernel for launches of wide waves: always instead of the register-staged tile
+    // kernel (dense blocks of 1,024 x 2,816 over 64 / 200 / 400 tokens 63 / 132 / 143 -> 34 / 41 /
+    // 46 us, clusters of 16 over 512 tokens 73 -> 70), and instead of the LDS ring where its
+    // 512-token workgroups leave the GPU unfilled and would split the contraction through memory
+    // (blocks of 1,536 x 4,096 over 512 / 1,000 tokens 404 / 412 -> 62 / 99 us, 64-neuron tiles of
+    // 8,192 inputs over 512 tokens 117 -> 95), or with 128-neuron tiles (1,536 x 4,096 over 4,096
+    // tokens 457 -> 301).  Launches of 32/64-neuron tiles that fill the GPU stay on the ring
+    // (64 tiles x 2,048 tokens 85 us, 87 here), and so do few tiles of very long rows on the
+    // register-staged kernel, whose split-K reaches 32 workgroups a tile (8,192 inputs, 8 / 16 /
+    // 32 tiles of 64 tokens: 18.5 / 17.1 / 21.5 us, 22.4 / 21.1 / 26.9 here; 4,096 inputs 17.0,
+    // 13.9 here).
+    for (auto &gp : groups) {
+        MfmaGroupExec &g = *gp;
+        uint64_t base = 0, tiles = 0;
+        uint32_t ksteps = 0;
+        bool ok = g.mt != 16u;
+        for (size_t m : g.members) {
+            const WaveExec &w = *waves[m];
+            ok = ok && w.rows_ok && w.xprod == 0u && w.rk_nb == waves[g.members[0]]->rk_nb &&
+                 w.rk_mis == waves[g.members[0]]->rk_mis;
+            base += (uint64_t)w.rows * (w.tokens / w.mt);
+            tiles += w.rk_tiles();
+            ksteps = std::max(ksteps, w.rk_ksteps);
+        }
+        g.rowsk = ok && (g.nt == 128u || (g.dma ? base < 256u : tiles > 64u || ksteps < 192u));
+        if (!g.rowsk) continue;
+        g.part_floats = 0;
+        for (size_t m : g.members) {
+            set_split(*waves[m], 1u);
+            use_rows(*waves[m], rows_waves(tiles, ksteps));
+        }
+    }
+    for (auto &w : waves) w->roff_h = {};
+    scratch_need = 0;
+    for (const auto &a : aux)
+        if (a->type == K44CmdType::ARGMAX_1D)
+            scratch_need = std::max(scratch_need, k44dev::argmax_scratch_floats(a->D, a->stride));
+    for (const auto &w : waves) scratch_need = std::max(scratch_need, w->part_floats);
     for (const auto &g : groups) scratch_need = std::max(scratch_need, g->part_floats);
 }
 
@@ -1216,7 +1254,8 @@ void K44GpuExecutorState::build_report() {
           << ", \"S\": " << w.S << ", \"cluster\": " << w.cluster << ", \"step\": " << w.step
           << ", \"tokens\": " << w.tokens << ", \"slab\": " << (w.mfma ? w.mt : w.slab)
           << ", \"U\": " << (w.mfma ? w.rows_per_stage : w.U)
-          << ", \"ksplit\": " << (w.mfma ? w.kgroups : w.ksplit)
+          << ", \"ksplit\": " << (w.rowsk ? w.rk_kw : w.mfma ? w.kgroups : w.ksplit)
+          << ", \"kernel\": \"" << (w.rowsk ? "rows" : w.path.substr(w.path.find('_') + 1u)) << "\""
           << ", \"sorted_segments\": " << (w.sorted_segments ? "true" : "false")
           << ", \"misaligned\": " << (w.misaligned ? "true" : "false")
           << ", \"phase_order\": " << (w.phase_order ? "true" : "false")

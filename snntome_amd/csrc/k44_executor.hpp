@@ -172,11 +172,15 @@ struct WaveExec {
     // launch never joins one of the fold's readers)
     std::vector<std::pair<uint64_t, uint64_t>> carry_rng;
     // Row-table MFMA kernel (k44_mfma_rows.hip): the positions of every index row as element
-    // offsets from rk_base, rk_kw waves per tile of 16 rk_nb neurons.
-    bool rowsk = false, rk_mis = false;
+    // offsets from rk_base, rk_kw waves per tile of 16 rk_nb neurons.  rows_ok: the kernel can run
+    // the wave (roff_h: its table); rowsk: it does (alone, or for MFMA waves in their group).
+    bool rows_ok = false, rowsk = false, rk_mis = false;
     uint32_t rk_nb = 0, rk_kw = 0, rk_subs = 0, rk_ksteps = 0, rk_B = 0, rk_vec = 1;
     uint64_t rk_base = 0;
+    std::vector<uint32_t> roff_h;
     DevBuf<uint32_t> roff;
+    uint32_t rk_ttiles() const { return tokens / 64u; }
+    uint64_t rk_tiles() const { return (uint64_t)rows * rk_subs * rk_ttiles(); }
     // 2-D spatial wave (VALU over the padded-plane tile layout): tile tables, output plane.
     bool tile2d = false;
     DevBuf<uint32_t> tile_x, tile_y;
@@ -195,6 +199,10 @@ struct MfmaGroupExec {
     std::vector<size_t> members;  // wave indices, plan order
     uint32_t nt = 0, mt = 0, rows = 0, items = 0, epi_items = 0, max_items = 0;
     bool dma = false, stream_loads = false, mis = false;
+    // every member runs on the row-table kernel: descriptors, workgroup columns and token tiles
+    bool rowsk = false;
+    DevBuf<k44dev::RowsArgs> rk_args;
+    uint32_t rk_cols = 0, rk_ttiles = 0;
     uint32_t prod = 0;  // product form (xprod) every member's gathers take
     k44dev::DmaShape dshape;
     size_t part_floats = 0;
@@ -305,6 +313,7 @@ struct K44GpuExecutorState {
     DevBuf<uint32_t> ids, history, step_ctr;  // token ids (EMBED / ARGMAX), greedy history
     DevBuf<float> in_stage;  // fp32 input channels on their way to the canvas (infer_f32)
     HostRing ring;           // outputs on their way to pageable host memory
+    std::recursive_mutex io;  // holds the ring: canvas reads of several threads stay independent
     uint32_t id_tokens = 0, hist_steps = 0;
     // Scratch shared by the commands of the plan (they run in order on one stream): split-K
     // partials of MFMA waves, per-chunk (value, index) partials of ARGMAX.
@@ -379,9 +388,13 @@ struct K44GpuExecutorState {
     static bool streaming_gather(const WaveExec &wx);
     void configure_mfma(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
                         size_t rows, uint32_t width);
-    bool configure_rows(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
-                        const std::vector<uint64_t> &starts, const std::vector<uint32_t> &tx,
-                        const std::vector<uint32_t> &ty);
+    bool rows_shape(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint64_t> &starts,
+                    const std::vector<uint32_t> &tx, const std::vector<uint32_t> &ty);
+    static uint32_t rows_waves(uint64_t tiles, uint32_t ksteps);
+    static void use_rows(WaveExec &wx, uint32_t kw);
+    k44dev::RowsArgs rows_args(const WaveExec &w, bool fused) const;
+    static void upload_fragments(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
+                                 size_t rows);
     void build_wave(const K44ExecCmd &c, WaveExec &wx);
     void build_wave2d(const K44ExecCmd &c, WaveExec &wx, const K44ResDesc &Lo,
                       const K44ResDesc &Li);
@@ -426,6 +439,7 @@ struct K44GpuExecutorState {
                            uint32_t items, uint32_t epi_items, bool dma, const k44dev::DmaShape &ds,
                            uint32_t prod, uint32_t max_items, bool mis,
                            const k44dev::NarrowPre &pre);
+    void launch_rows(const WaveExec &w);
     void launch_mfma(const WaveExec &w);
     void launch_group(const MfmaGroupExec &g);
     void launch_wave(const WaveExec &w);

@@ -114,7 +114,7 @@ __device__ __forceinline__ void rows_finish(const RowsArgs &a, const float *red,
 }  // namespace
 
 template <int NB, int KW, bool MIS>
-__global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(RowsArgs a) {
+__global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(RowsLaunch l) {
     constexpr int NW = KW == 1 ? 4 : KW;
     constexpr int SLOTS = 4;                       // partial sums met in LDS at a time
     constexpr int RED = KW == 1 ? 0 : SLOTS * NB * 16 * RP * 4;
@@ -122,15 +122,25 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
     __shared__ __attribute__((aligned(16))) char smem[SMEM];
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t col = blockIdx.x;
+    RowsArgs a = l.one;
+    if (l.n) {
+        const kconst_u32 *start = (const kconst_u32 *)l.start;
+        uint32_t w = 0;
+        while (w + 1u < l.n && col >= start[w + 1u]) ++w;
+        col -= start[w];
+        a = l.waves[w];
+    }
     const uint32_t tile = KW == 1 ? blockIdx.y * 4u + (uint32_t)wave : blockIdx.y;
-    if (KW == 1 && tile >= a.ttiles) return;  // (no workgroup barrier with KW = 1)
-    const uint32_t sub = blockIdx.x, row = sub / a.subs;
+    if (tile >= a.ttiles) return;  // whole workgroup, or a wave of one without barriers (KW = 1)
+    const uint32_t row = col / a.subs, blk = (col - row * a.subs) * NB;
     const uint32_t k0 = KW == 1 ? 0u : (uint32_t)wave;
     _Float16(*xs)[PITCH] = reinterpret_cast<_Float16(*)[PITCH]>(smem + wave * XS_BYTES);
 
     const int gr = lane >> 3, gc = (lane & 7) * 8;  // gather: rows 4 gr .. +3, tokens gc .. +7
     const u4_t *roff = reinterpret_cast<const u4_t *>(a.roff + (uint64_t)row * a.ksteps * 32u) + gr;
-    const h8_t *wf = reinterpret_cast<const h8_t *>(a.Wf) + (uint64_t)sub * a.ksteps * NB * 64u + lane;
+    const h8_t *wf = reinterpret_cast<const h8_t *>(a.Wf) +
+                     ((uint64_t)row * a.ksteps * a.blocks + blk) * 64u + lane;
     const uint32_t tx = (a.tile_x ? a.tile_x[tile] : 64u * tile) + (uint32_t)gc;
     const __half *xt = a.X + tx;
     // MIS: element offset of the lane's tokens past the 16-byte boundary below them
@@ -160,7 +170,7 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
     };
     auto load_a = [&](uint32_t ks) {
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) ar[nb] = wf[((uint64_t)ks * NB + nb) * 64u];
+        for (int nb = 0; nb < NB; ++nb) ar[nb] = wf[((uint64_t)ks * a.blocks + nb) * 64u];
     };
     const int tr_row = 8 * (lane >> 4) + ((lane & 15) >> 2), tr_col = 4 * (lane & 3);
     if (k0 < a.ksteps) {
@@ -179,7 +189,9 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
             h8_t af[NB];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) af[nb] = ar[nb];
-            // next step in flight (past the end: the last step again, unused)
+            // Next step in flight (past the end: the last step again, unused).  Two steps in
+            // flight need 184 registers instead of 128 and were slower for it (4,096 x 512
+            // scattered 7.0 us instead of 6.1, a dense block over 512 tokens 67 instead of 58).
             load_a(min(ks + KW, a.ksteps - 1u));
             load_x(rn);
             rn = roff[(uint64_t)min(ks + 2u * KW, a.ksteps - 1u) * 8u];
@@ -196,7 +208,7 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
         }
     }
 
-    const uint32_t j0 = sub * 16u * NB;
+    const uint32_t j0 = (row * a.blocks + blk) * 16u;
     const uint64_t ty = a.tile_y ? (uint64_t)a.tile_y[tile] : 64ull * tile;
     const int g = lane >> 4, c = lane & 15;
     if constexpr (KW == 1) {
@@ -236,36 +248,36 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
 }
 
 template <int NB, int KW>
-static hipError_t launch_rows_kw(const RowsArgs &a, uint32_t rows, bool mis, hipStream_t stream) {
-    const uint32_t gy = KW == 1 ? (a.ttiles + 3u) / 4u : a.ttiles;
-    const dim3 grid(rows * a.subs, gy, 1u), block(64u * (KW == 1 ? 4u : KW), 1u, 1u);
+static hipError_t launch_rows_kw(const RowsLaunch &l, uint32_t cols, uint32_t ttiles, bool mis,
+                                 hipStream_t stream) {
+    const dim3 grid(cols, KW == 1 ? (ttiles + 3u) / 4u : ttiles, 1u);
+    const dim3 block(64u * (KW == 1 ? 4u : KW), 1u, 1u);
     if (mis)
-        hipLaunchKernelGGL((k44_mfma_rows_kernel<NB, KW, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((k44_mfma_rows_kernel<NB, KW, true>), grid, block, 0, stream, l);
     else
-        hipLaunchKernelGGL((k44_mfma_rows_kernel<NB, KW, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((k44_mfma_rows_kernel<NB, KW, false>), grid, block, 0, stream, l);
     return hipGetLastError();
 }
 
 template <int NB>
-static hipError_t launch_rows_nb(const RowsArgs &a, uint32_t rows, uint32_t kw, bool mis,
-                                 hipStream_t stream) {
-    if (kw == 8u) return launch_rows_kw<NB, 8>(a, rows, mis, stream);
-    if (kw == 4u) return launch_rows_kw<NB, 4>(a, rows, mis, stream);
-    if (kw == 1u) return launch_rows_kw<NB, 1>(a, rows, mis, stream);
+static hipError_t launch_rows_nb(const RowsLaunch &l, uint32_t cols, uint32_t ttiles, uint32_t kw,
+                                 bool mis, hipStream_t stream) {
+    if (kw == 8u) return launch_rows_kw<NB, 8>(l, cols, ttiles, mis, stream);
+    if (kw == 4u) return launch_rows_kw<NB, 4>(l, cols, ttiles, mis, stream);
+    if (kw == 1u) return launch_rows_kw<NB, 1>(l, cols, ttiles, mis, stream);
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_mfma_rows(const RowsArgs &a, uint32_t rows, uint32_t nb, uint32_t kw, bool mis,
-                            hipStream_t stream) {
-    if (rows == 0u || a.ttiles == 0u) return hipSuccess;
-    if (a.ksteps == 0u || a.subs == 0u || (uint64_t)rows * a.subs > 0x7fffffffull ||
-        (kw == 1u ? (a.ttiles + 3u) / 4u : a.ttiles) > 65535u)
+hipError_t launch_mfma_rows(const RowsLaunch &l, uint32_t cols, uint32_t ttiles, uint32_t nb,
+                            uint32_t kw, bool mis, hipStream_t stream) {
+    if (cols == 0u || ttiles == 0u) return hipSuccess;
+    if (cols > 0x7fffffffu || (kw == 1u ? (ttiles + 3u) / 4u : ttiles) > 65535u)
         return hipErrorInvalidValue;
     switch (nb) {
-    case 1u: return launch_rows_nb<1>(a, rows, kw, mis, stream);
-    case 2u: return launch_rows_nb<2>(a, rows, kw, mis, stream);
-    case 3u: return launch_rows_nb<3>(a, rows, kw, mis, stream);
-    case 4u: return launch_rows_nb<4>(a, rows, kw, mis, stream);
+    case 1u: return launch_rows_nb<1>(l, cols, ttiles, kw, mis, stream);
+    case 2u: return launch_rows_nb<2>(l, cols, ttiles, kw, mis, stream);
+    case 3u: return launch_rows_nb<3>(l, cols, ttiles, kw, mis, stream);
+    case 4u: return launch_rows_nb<4>(l, cols, ttiles, kw, mis, stream);
     default: return hipErrorInvalidValue;
     }
 }

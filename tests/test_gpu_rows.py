@@ -117,3 +117,52 @@ def test_image_convolutions(wavec, orc, tuning, kw, frames, H, W, cin, cout, res
     halo = np.ones(cout * lay.channel_stride, bool)
     halo[lay.offsets(cout).ravel()] = False
     assert not out[halo].any()
+
+
+@pytest.mark.parametrize("tile,tokens", [(64, 100), (64, 512), (32, 200)])
+def test_grouped_dense_tiles(wavec, orc, tile, tokens):
+    """Sub-waves of a pruned projection (dense tiles, several row lengths, outputs through
+    cout_map) share one row-table launch; the launch equals its commands run one by one bit for
+    bit and the per-neuron oracle within tolerance."""
+    rng = np.random.default_rng(tile + tokens)
+    n_cl, K, S, cout = 4, 2, 64, 1000
+    C = n_cl * S
+    pick = np.argsort(rng.random((cout, n_cl)), axis=1)[:, :K]
+    starts = (pick * S).astype(np.uint32)
+    w = synth.normal_f16(rng, (cout, K * S), 0.1)
+    b = synth.normal_f16(rng, (cout,), 0.1)
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", C, 1, tokens, is_1d=True)
+    g.add_pruned_wave("p", "x", "y", starts, S, w, b, tile=tile, act="silu")
+    plan = g.compile()
+    plan.init_gpu()
+    rep = plan.exec_report()
+    assert {r["kernel"] for r in rep["waves"]} == {"rows"} and len(rep["waves"]) >= 2
+    assert len(rep["groups"]) == 1 and rep["launches_per_run"] == 1
+    plan.fill_input_uniform(7)
+    plan.execute(1)
+    st = stride_of(tokens)
+    x0, y0 = int(plan.cmds[0]["src_off"]), int(plan.cmds[0]["y_off"])
+    canvas = plan.read_canvas(0, int(plan.summary["canvas_elems"]))
+    plan.write_canvas(y0, np.zeros(cout * st, np.uint16))
+    plan.execute_range(0, len(plan.cmds))
+    assert np.array_equal(plan.read_canvas(y0, cout * st), canvas[y0:y0 + cout * st])
+    ref = orc.wave_f64(canvas, (x0 + starts.astype(np.uint64) * st).ravel(), w, b, None, K, S, 1,
+                       st, st, st, "silu")
+    y = canvas[y0:y0 + cout * st].view(np.float16).reshape(cout, st).astype(np.float64)
+    assert orc.rel_err(y[:, :tokens], ref[:, :tokens]) <= TOL
+
+
+def test_long_rows_keep_their_split(wavec):
+    """Few tiles of very long rows stay on the register-staged kernel, wider ones do not."""
+    kernels = {}
+    for tokens in (64, 320):
+        g = wavec.WaveGraph(kv_cache_max_seq=0)
+        g.add_input("x", 8192, 1, tokens, is_1d=True)
+        g.add_cluster_wave("w", "x", "y", np.zeros((16, 16), np.uint32), 512,
+                           np.zeros((16 * 64, 8192), np.float16), None, cluster=64)
+        plan = g.compile()
+        plan.init_gpu()
+        kernels[tokens] = plan.exec_report()["waves"][0]["kernel"]
+        plan.release_gpu()
+    assert kernels == {64: "tile", 320: "rows"}
