@@ -280,6 +280,92 @@ __global__ __launch_bounds__(1024) void k44_rmsnorm_regs_kernel(__half *__restri
     }
 }
 
+// Middling token counts (65 .. 8,191): workgroup = 8 tokens x 1,024 channel lanes, each thread's
+// channels in registers from the sum to the store, so the input is read once.  Bound by the
+// gather of 16-byte row pieces: workgroup b works for XCD b % 8 (round-robin dispatch) on a
+// contiguous run of octets, so the 8 octets of a 128-byte line meet in one L2 instead of being
+// fetched by every XCD.  Sums of squares in 64-bit floats (each square is exact in it): 3
+// instructions an element instead of the 25 of the integer limbs that the decode kernels need to
+// be independent of the order.  2,048 tokens x 2,048 channels: 26.8 -> 9.4 us, 200 x
+// 1,024 5.5 -> 4.9.
+__device__ __forceinline__ double shfl_xor_f64(double v, int m) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)b, m, 64);
+    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(b >> 32), m, 64);
+    return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+template <int CPT>
+__global__ __launch_bounds__(1024) void k44_rmsnorm_octet_kernel(__half *__restrict__ y,
+                                                                 const __half *__restrict__ x,
+                                                                 const __half *__restrict__ gamma,
+                                                                 uint32_t D, uint32_t stride,
+                                                                 float eps) {
+    __shared__ double part[16][8];
+    __shared__ float inv_s[8];
+    const uint32_t n = gridDim.x, xcd = blockIdx.x & 7u, q = n >> 3, r = n & 7u;
+    const uint32_t t0 = (xcd * q + min(xcd, r) + (blockIdx.x >> 3)) * 8u;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint16_t *g16 = reinterpret_cast<const uint16_t *>(gamma ? gamma : x);
+    uint4 v[CPT];
+    uint32_t gv[CPT];
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {  // all loads together, without branches around them
+        const uint32_t c = tid + (uint32_t)u * 1024u, cc = c < D ? c : D - 1u;
+        const uint4 t = *reinterpret_cast<const uint4 *>(x + (uint64_t)cc * stride + t0);
+        gv[u] = g16[cc];
+        v[u] = c < D ? t : uint4{0u, 0u, 0u, 0u};
+    }
+    double ss[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+        const __half *h = reinterpret_cast<const __half *>(&v[u]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const double f = (double)__half2float(h[k]);
+            ss[k] = fma(f, f, ss[k]);
+        }
+    }
+    // Wave sums: at each of the first three steps a lane hands over half of its tokens, so lane l
+    // ends with token 4 (l & 1) + 2 (l >> 1 & 1) + (l >> 2 & 1) summed over 8 lanes; then plain.
+#pragma unroll
+    for (int m = 1, w = 4; m < 8; m <<= 1, w >>= 1) {
+        const bool up = (lane & (uint32_t)m) != 0u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k >= w) continue;
+            const double keep = up ? ss[k + w] : ss[k], give = up ? ss[k] : ss[k + w];
+            ss[k] = keep + shfl_xor_f64(give, m);
+        }
+    }
+#pragma unroll
+    for (int m = 8; m < 64; m <<= 1) ss[0] += shfl_xor_f64(ss[0], m);
+    if (lane < 8u) part[wave][4u * (lane & 1u) + (lane & 2u) + (lane >> 2)] = ss[0];
+    __syncthreads();
+    if (tid < 8u) {
+        double t = part[0][tid];
+#pragma unroll
+        for (int w = 1; w < 16; ++w) t += part[w][tid];
+        inv_s[tid] = rsqrtf((float)t / (float)D + eps);
+    }
+    __syncthreads();
+    float inv[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) inv[k] = inv_s[k];
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+        const uint32_t c = tid + (uint32_t)u * 1024u;
+        if (c >= D) break;
+        const __half *h = reinterpret_cast<const __half *>(&v[u]);
+        const float g = gamma ? __half2float(__ushort_as_half((unsigned short)gv[u])) : 1.0f;
+        uint4 o;
+        __half *oh = reinterpret_cast<__half *>(&o);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) oh[k] = norm_scale(h[k], inv[k], g);
+        *reinterpret_cast<uint4 *>(y + (uint64_t)c * stride + t0) = o;
+    }
+}
+
 // Prefill RMSNorm with the token shift of its output fused (k44_rmsnorm_regs_kernel followed by
 // k44_token_shift_prefill_kernel, the same operations in the same order, so the same values).
 // The workgroup of 32 tokens also sums the squares of the HK = 4 tokens before its block (the
@@ -941,6 +1027,26 @@ hipError_t launch_rmsnorm(__half *y, const __half *x, const __half *gamma, uint3
             K44_RMSW(16);
         }
 #undef K44_RMSW
+        return hipGetLastError();
+    }
+    // Rows of more than one 64-token tile (decode norms, whose exact sums meet those of folded
+    // producers, keep the kernel below), channels within 8 per thread; below 768 channels most of
+    // the 1,024 lanes idle (512 x 4,096 tokens 7.7 us below, 8.3 here; 768: 11.6 and 9.1).
+    if (!shift && !slots && stride > 64u && D >= 768u && D <= 8u * 1024u) {
+        const uint32_t cpt = (D + 1023u) / 1024u;
+#define K44_RMSO(C)                                                                              \
+    hipLaunchKernelGGL((k44_rmsnorm_octet_kernel<C>), dim3(octets), dim3(1024), 0, stream, y, x,  \
+                       gamma, D, stride, eps)
+        if (cpt == 1u) {
+            K44_RMSO(1);
+        } else if (cpt == 2u) {
+            K44_RMSO(2);
+        } else if (cpt <= 4u) {
+            K44_RMSO(4);
+        } else {
+            K44_RMSO(8);
+        }
+#undef K44_RMSO
         return hipGetLastError();
     }
     const dim3 grid(chunks, (D + cslice - 1u) / cslice);
