@@ -13,9 +13,9 @@
 // ...) and add their accumulators in LDS, in a fixed order: the chain of dependent gathers is
 // KW times shorter and no partial sums leave the workgroup.  KW = 1 gives each of 4 waves a
 // 64-token tile of its own (same A fragments through L1) once there are enough tiles.
-// 4,096 neurons in clusters of 64, 512 scattered synapses, 256 tokens: 17.7, 6.8 and 6.1 us with
-// KW = 1, 4 and 8 (33 MB of gathers and weights: 5.4 TB/s from L2); 16 synapses over 4,096
-// tokens: 5.6 us.
+// The token tiles of one neuron tile share its weights, through one XCD's L2: in grid order when
+// the columns are a multiple of 8, else with the items numbered column by column and each XCD
+// taking a contiguous run of them.
 #include <algorithm>
 
 #include "k44_mfma_rows.hpp"
@@ -122,7 +122,12 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
     __shared__ __attribute__((aligned(16))) char smem[SMEM];
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    uint32_t col = blockIdx.x;
+    uint32_t col = blockIdx.x, ty0 = blockIdx.y;
+    if (l.by_cols) {
+        const uint32_t item = xcd_contiguous(blockIdx.x, gridDim.x);
+        col = item / l.by_cols;
+        ty0 = item - col * l.by_cols;
+    }
     RowsArgs a = l.one;
     if (l.n) {
         const kconst_u32 *start = (const kconst_u32 *)l.start;
@@ -131,7 +136,7 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
         col -= start[w];
         a = l.waves[w];
     }
-    const uint32_t tile = KW == 1 ? blockIdx.y * 4u + (uint32_t)wave : blockIdx.y;
+    const uint32_t tile = KW == 1 ? ty0 * 4u + (uint32_t)wave : ty0;
     if (tile >= a.ttiles) return;  // whole workgroup, or a wave of one without barriers (KW = 1)
     const uint32_t row = col / a.subs, blk = (col - row * a.subs) * NB;
     const uint32_t k0 = KW == 1 ? 0u : (uint32_t)wave;
@@ -248,9 +253,11 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
 }
 
 template <int NB, int KW>
-static hipError_t launch_rows_kw(const RowsLaunch &l, uint32_t cols, uint32_t ttiles, bool mis,
+static hipError_t launch_rows_kw(RowsLaunch l, uint32_t cols, uint32_t ttiles, bool mis,
                                  hipStream_t stream) {
-    const dim3 grid(cols, KW == 1 ? (ttiles + 3u) / 4u : ttiles, 1u);
+    const uint32_t tys = KW == 1 ? (ttiles + 3u) / 4u : ttiles;
+    l.by_cols = cols % 8u != 0u && tys > 1u && cols > 8u ? tys : 0u;
+    const dim3 grid = l.by_cols ? dim3(cols * tys, 1u, 1u) : dim3(cols, tys, 1u);
     const dim3 block(64u * (KW == 1 ? 4u : KW), 1u, 1u);
     if (mis)
         hipLaunchKernelGGL((k44_mfma_rows_kernel<NB, KW, true>), grid, block, 0, stream, l);
@@ -271,7 +278,7 @@ static hipError_t launch_rows_nb(const RowsLaunch &l, uint32_t cols, uint32_t tt
 hipError_t launch_mfma_rows(const RowsLaunch &l, uint32_t cols, uint32_t ttiles, uint32_t nb,
                             uint32_t kw, bool mis, hipStream_t stream) {
     if (cols == 0u || ttiles == 0u) return hipSuccess;
-    if (cols > 0x7fffffffu || (kw == 1u ? (ttiles + 3u) / 4u : ttiles) > 65535u)
+    if ((uint64_t)cols * ttiles > 0x7fffffffull || (kw == 1u ? (ttiles + 3u) / 4u : ttiles) > 65535u)
         return hipErrorInvalidValue;
     switch (nb) {
     case 1u: return launch_rows_nb<1>(l, cols, ttiles, kw, mis, stream);

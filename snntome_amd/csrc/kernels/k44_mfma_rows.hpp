@@ -4,6 +4,12 @@
 
 namespace k44dev {
 
+// Item of workgroup b of n: workgroups go round-robin over the 8 XCDs, each takes a contiguous run.
+__device__ __forceinline__ uint32_t xcd_contiguous(uint32_t b, uint32_t n) {
+    const uint32_t x = b & 7u, q = n >> 3, r = n & 7u;
+    return x * q + min(x, r) + (b >> 3);
+}
+
 struct RowsArgs {
     const __half *X;       // canvas + the wave's lowest row offset
     const uint32_t *roff;  // [index rows][32 ksteps] element offset of every position from X
@@ -30,6 +36,7 @@ struct RowsLaunch {
     const RowsArgs *waves = nullptr;
     const uint32_t *start = nullptr;
     uint32_t n = 0;
+    uint32_t by_cols = 0;  // token tiles when items are numbered column by column (launcher)
     RowsArgs one{};
 };
 

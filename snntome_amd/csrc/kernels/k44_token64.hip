@@ -8,9 +8,12 @@
 // the RDNA4 WMMA vector order (k44_plan_types.hpp convert_raw_to_wmma), bias always added,
 //     Y[t][j][m] = fp16_round_toward_zero(bias[j] + sum_k W[j][k] * X[t][idx[j/cluster][k]][m]).
 //
-// MI355X mapping.  One wave = one 64-token tile x 16*NB neurons of one cluster (NB = 4, 2, 1:
+// MI355X mapping.  One wave = one 64-token tile x 16*NB neurons of one cluster (NB = 4, 3, 2, 1:
 // the widest that divides the cluster); a workgroup holds 4 waves on 4 consecutive tiles (same
-// neurons, so the A fragments are shared through L1).  Per 32-deep k-step the wave gathers its
+// neurons, so the A fragments are shared through L1), or, while such tiles are too few to fill
+// the GPU, KW waves on one tile that share its k-steps (k = wave, wave + KW, ...) and add their
+// sums in LDS in a fixed order: one tile x 2,048 neurons of 512 inputs 16.1 -> 6.2 us, 5 tiles
+// x 4,080 neurons in clusters of 48 (three blocks a wave instead of one) 22.9 -> 13.1 us.  Per 32-deep k-step the wave gathers its
 // 32 index rows (128 bytes each, 8 lanes x 16 bytes per row) into a private LDS tile, and the B
 // operand of v_mfma_f32_16x16x32_f16 comes out with ds_read_b64_tr_b16 (8 positions of one
 // token per lane), exactly as in the dense-cluster tile kernel.  A fragments are read straight
@@ -24,17 +27,28 @@
 
 #include "k44_launch.hpp"
 #include "k44_mfma_dma.hpp"
+#include "k44_mfma_rows.hpp"
 
 namespace k44dev {
 
-template <int NB>
-__global__ __launch_bounds__(256) void k44_token64_kernel(Token64Args a) {
+template <int NB, int KW>
+__global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_token64_kernel(Token64Args a) {
     constexpr int PITCH = 72;  // halves per LDS row: 64 tokens + 16-byte skew
-    __shared__ __attribute__((aligned(16))) _Float16 xs[4][32][PITCH];
-    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
-    const uint32_t tile = blockIdx.y * 4u + (uint32_t)wave;
-    if (tile >= a.tiles) return;  // no workgroup barrier in this kernel
-    const uint32_t j0 = blockIdx.x * 16u * NB;
+    constexpr int NW = KW == 1 ? 4 : KW, XS = 32 * PITCH * 2;
+    constexpr int RP = 68;     // floats per neuron of the sums that meet in LDS
+    constexpr int RED = KW == 1 ? 0 : 4 * NB * 16 * RP * 4;
+    __shared__ __attribute__((aligned(16))) char smem[NW * XS > RED ? NW * XS : RED];
+    const int lane = (int)(threadIdx.x & 63u);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    _Float16(*xs)[PITCH] = reinterpret_cast<_Float16(*)[PITCH]>(smem + wave * XS);
+    // KW > 1 (1-D grid): the tiles of one block of neurons are neighbours in one XCD's contiguous
+    // run of items, so its weights come through one L2 (8 tiles x 4,080
+    // neurons in clusters of 48: 20.6 us in grid order, 15.6 so).
+    const uint32_t item = KW == 1 ? 0u : xcd_contiguous(blockIdx.x, gridDim.x);
+    const uint32_t tile = KW == 1 ? blockIdx.y * 4u + (uint32_t)wave : item % a.tiles;
+    if (KW == 1 && tile >= a.tiles) return;  // no workgroup barrier with KW = 1
+    const uint32_t k0 = KW == 1 ? 0u : (uint32_t)wave;
+    const uint32_t j0 = (KW == 1 ? blockIdx.x : item / a.tiles) * 16u * NB;
     const uint32_t B = a.B_vec16 * 16u;
     const uint32_t ksteps = (a.B_vec16 + 1u) / 2u;
     const uint32_t *irow = a.idx + (uint64_t)(j0 / a.cluster) * B;
@@ -47,7 +61,7 @@ __global__ __launch_bounds__(256) void k44_token64_kernel(Token64Args a) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         f4_t b0 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (a.bias) {
+        if (a.bias && wave * (KW - 1) == 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) b0[i] = __half2float(a.bias[j0 + 16u * nb + 4u * g + i]);
         }
@@ -82,28 +96,30 @@ __global__ __launch_bounds__(256) void k44_token64_kernel(Token64Args a) {
     uint32_t ia[4], ib[4];
     u4_t xr[4];
     h8_t ar[NB];
-    load_idx(0u, ia);
-    load_idx(min(1u, ksteps - 1u), ib);
-    load_x(ia, xr);
-    load_a(0u, ar);
     const int tr_row = 8 * g + ((lane & 15) >> 2), tr_col = 4 * (lane & 3);
-    for (uint32_t ks = 0; ks < ksteps; ++ks) {
+    if (k0 < ksteps) {
+        load_idx(k0, ia);
+        load_a(k0, ar);
+        load_idx(min(k0 + KW, ksteps - 1u), ib);
+        load_x(ia, xr);
+    }
+    for (uint32_t ks = k0; ks < ksteps; ks += KW) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<u4_t *>(&xs[wave][8 * i + gr][gc]) = xr[i];
+            *reinterpret_cast<u4_t *>(&xs[8 * i + gr][gc]) = xr[i];
         h8_t af[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) af[nb] = ar[nb];
         // Next k-step in flight (clamped at the end: a re-read of the last step, unused).
-        const uint32_t kn = min(ks + 1u, ksteps - 1u);
+        const uint32_t kn = min(ks + KW, ksteps - 1u);
 #pragma unroll
         for (int i = 0; i < 4; ++i) ia[i] = ib[i];
-        load_idx(min(ks + 2u, ksteps - 1u), ib);
+        load_idx(min(ks + 2u * KW, ksteps - 1u), ib);
         load_x(ia, xr);
         load_a(kn, ar);
 #pragma unroll
         for (int tb = 0; tb < 4; ++tb) {
-            const _Float16 *p = &xs[wave][tr_row][tr_col + 16 * tb];
+            const _Float16 *p = &xs[tr_row][tr_col + 16 * tb];
             const h4_t lo = lds_read_tr16(p);
             const h4_t hi = lds_read_tr16(p + 4 * PITCH);
             const h8_t b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -114,14 +130,66 @@ __global__ __launch_bounds__(256) void k44_token64_kernel(Token64Args a) {
     }
 
     // C layout: lane holds C[4g + i][lane & 15] of every 16x16 tile; round toward zero.
-    __half *yt = a.Y + ((uint64_t)tile * a.Cout + j0) * 64u + (lane & 15);
+    if constexpr (KW == 1) {
+        __half *yt = a.Y + ((uint64_t)tile * a.Cout + j0) * 64u + (lane & 15);
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int tb = 0; tb < 4; ++tb)
-                yt[(uint64_t)(16 * nb + 4 * g + i) * 64u + 16u * tb] = __float2half_rz(acc[nb][tb][i]);
+                for (int tb = 0; tb < 4; ++tb)
+                    yt[(uint64_t)(16 * nb + 4 * g + i) * 64u + 16u * tb] =
+                        __float2half_rz(acc[nb][tb][i]);
+        return;
+    }
+    __syncthreads();  // every wave is done with its k-step region
+    if constexpr (KW == 8) {  // waves 4..7 add theirs to waves 0..3
+        f4_t *ex = reinterpret_cast<f4_t *>(smem) + (wave & 3) * NB * 256 + lane;
+        if (wave >= 4)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) ex[(nb * 4 + tb) * 64] = acc[nb][tb];
+        __syncthreads();
+        if (wave < 4)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[nb][tb] += ex[(nb * 4 + tb) * 64];
+        __syncthreads();
+    }
+    float *red = reinterpret_cast<float *>(smem);
+    if (wave < 4) {
+        float *ws = red + wave * NB * 16 * RP;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb)
+                    ws[(16 * nb + 4 * g + i) * RP + 16 * tb + (lane & 15)] = acc[nb][tb][i];
+    }
+    __syncthreads();
+    __half *yt = a.Y + ((uint64_t)tile * a.Cout + j0) * 64u;
+    for (int u = (int)threadIdx.x; u < NB * 128; u += 64 * NW) {  // (neuron, 8-token chunk)
+        const int n = u >> 3, t0 = 8 * (u & 7);
+        u4_t o;
+        __half *oh = reinterpret_cast<__half *>(&o);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float v = red[n * RP + t0 + e];
+#pragma unroll
+            for (int s = 1; s < 4; ++s) v += red[(s * NB * 16 + n) * RP + t0 + e];
+            oh[e] = __float2half_rz(v);
+        }
+        __half *dst = yt + (uint64_t)n * 64u + t0;
+        if (reinterpret_cast<uintptr_t>(a.Y) % 16u == 0u) {
+            *reinterpret_cast<u4_t *>(dst) = o;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dst[e] = oh[e];
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -322,14 +390,35 @@ hipError_t launch_token64(const Token64Args &a, hipStream_t stream, int ring_mod
         return hipGetLastError();
     }
     const uint32_t c16 = a.cluster / 16u;
-    const int nb = c16 % 4u == 0u ? 4 : (c16 % 2u == 0u ? 2 : 1);
-    const dim3 grid(a.Cout / (16u * (uint32_t)nb), (a.tiles + 3u) / 4u, 1u), block(256u, 1u, 1u);
-    if (nb == 4)
-        hipLaunchKernelGGL(k44_token64_kernel<4>, grid, block, 0, stream, a);
-    else if (nb == 2)
-        hipLaunchKernelGGL(k44_token64_kernel<2>, grid, block, 0, stream, a);
-    else
-        hipLaunchKernelGGL(k44_token64_kernel<1>, grid, block, 0, stream, a);
+    uint32_t nb = c16 % 4u == 0u ? 4u : c16 % 3u == 0u ? 3u : c16 % 2u == 0u ? 2u : 1u;
+    // Waves per tile: 8 while there is at most a tile per CU (one tile x 2,048 neurons 6.5 us, 7.4
+    // with 4; 3 tiles x 8,192 neurons of 1,024 inputs 19.8, 16.2 with 4), 4 until the tiles
+    // give 6 waves per CU by themselves, 1 for rows of under 4 k-steps (64 inputs: 4.6 us, 5.2
+    // with 4; and 2 blocks per wave rather than 3: 3,456 neurons of 96 inputs, 2 tiles, 5.8 and
+    // 7.1); with a forced mode, the one-wave kernel whose sums the ring kernels repeat.
+    const uint32_t ksteps = (a.B_vec16 + 1u) / 2u;
+    if (nb == 3u && ksteps < 4u) nb = c16 % 2u == 0u ? 2u : 1u;
+    const uint64_t wgs = (uint64_t)(a.Cout / (16u * nb)) * a.tiles;
+    const uint32_t kw = ring_mode >= 0 || wgs >= 1536u || ksteps < 4u ? 1u
+                        : ksteps >= 8u && wgs <= 256u                 ? 8u
+                                                                      : 4u;
+    const dim3 grid = kw == 1u ? dim3(a.Cout / (16u * nb), (a.tiles + 3u) / 4u, 1u)
+                               : dim3((uint32_t)wgs, 1u, 1u);
+    const dim3 block(kw == 1u ? 256u : 64u * kw, 1u, 1u);
+#define K44_T64(NB)                                                                              \
+    if (kw == 8u)                                                                                \
+        hipLaunchKernelGGL((k44_token64_kernel<NB, 8>), grid, block, 0, stream, a);              \
+    else if (kw == 4u)                                                                           \
+        hipLaunchKernelGGL((k44_token64_kernel<NB, 4>), grid, block, 0, stream, a);              \
+    else                                                                                         \
+        hipLaunchKernelGGL((k44_token64_kernel<NB, 1>), grid, block, 0, stream, a);
+    switch (nb) {
+    case 4u: K44_T64(4) break;
+    case 3u: K44_T64(3) break;
+    case 2u: K44_T64(2) break;
+    default: K44_T64(1) break;
+    }
+#undef K44_T64
     return hipGetLastError();
 }
 

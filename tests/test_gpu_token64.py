@@ -144,3 +144,21 @@ def test_token64_64bit_substrate(wavec, orc, batch):
         err = orc.rel_err(y[t], ref)
         _log(f"[token64 64-bit batch={batch} tile {t}] rel err {err:.3e}")
         assert err <= TOL
+
+
+@pytest.mark.parametrize("cluster,B_vec16,batch", [
+    (48, 7, 64), (96, 8, 200), (16, 16, 20), (32, 17, 130), (64, 33, 70), (80, 9, 64), (48, 300, 64),
+    (96, 6, 100)])
+def test_token64_shared_k_steps(wavec, orc, cluster, B_vec16, batch):
+    """Few tiles: 4 or 8 waves share a tile's k-steps (rows of 4 to 150 k-steps, half-empty last
+    ones, three-block clusters), and rows of under 4 k-steps that one wave runs alone."""
+    err = _token64_case(wavec, orc, Cin=2000, Cout=cluster * 3, cluster=cluster, B_vec16=B_vec16,
+                        batch=batch, seed=cluster + B_vec16, bad_index=B_vec16 == 9)
+    assert err <= TOL
+
+
+def test_token64_many_tiles_of_odd_clusters(wavec, orc):
+    """Enough tiles for one wave each, three 16-neuron blocks per wave."""
+    err = _token64_case(wavec, orc, Cin=800, Cout=48 * 64, cluster=48, B_vec16=8, batch=64 * 25,
+                        seed=5)
+    assert err <= TOL
