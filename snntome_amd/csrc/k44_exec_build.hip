@@ -298,13 +298,13 @@ bool K44GpuExecutorState::rows_shape(const K44ExecCmd &c, WaveExec &wx,
     return true;
 }
 
-// Waves per tile: 8 (4 for short rows), 4 once there are 512 tiles of 64 tokens (64 neuron tiles
-// of 8,192 inputs over 512 tokens, rows from HBM: 110 us with 8, 88 with 4; 64 x 8 tiles of 600
-// scattered inputs 11.1 and 10.7), 1 once the tiles alone give 6 waves per CU (64 x 16 tiles: 20.8
-// us with 4, 23.3 with 1; twice the tiles: 57 and 44).
+// Waves per tile: 8 (4 for short rows) while there is at most a tile of 64 tokens per CU (64 x 4
+// tiles of 512 scattered inputs 6.1 us, 6.8 with 4; 64 x 8 tiles of 8,192 inputs, rows from HBM,
+// 110 us, 88 with 4; of 600 scattered inputs 11.1 and 10.7), then 4, and 1 once the tiles alone
+// give 6 waves per CU (64 x 16 tiles: 20.8 us with 4, 23.3 with 1; twice the tiles: 57 and 44).
 uint32_t K44GpuExecutorState::rows_waves(uint64_t tiles, uint32_t ksteps) {
     if (tune(Tune::Rows) > 0) return (uint32_t)tune(Tune::Rows);
-    return tiles >= 1536u ? 1u : ksteps >= 8u && tiles < 512u ? 8u : 4u;
+    return tiles >= 1536u ? 1u : ksteps >= 8u && tiles <= 256u ? 8u : 4u;
 }
 
 void K44GpuExecutorState::use_rows(WaveExec &wx, uint32_t kw) {

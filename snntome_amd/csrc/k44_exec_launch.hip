@@ -152,7 +152,7 @@ void K44GpuExecutorState::launch_group(const MfmaGroupExec &g) {
     if (g.rowsk) {
         const WaveExec &w = *waves[g.members[0]];
         k44dev::RowsLaunch l;
-        if (g.members.size() > 1u) {
+            if (g.members.size() > 1u) {
             l.waves = g.rk_args.p;
             l.start = g.start.p;
             l.n = (uint32_t)g.members.size();
