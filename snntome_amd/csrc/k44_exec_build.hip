@@ -298,6 +298,110 @@ bool K44GpuExecutorState::rows_shape(const K44ExecCmd &c, WaveExec &wx,
     return true;
 }
 
+// Job tiles of a wave whose neurons have segments of their own: the (neuron, segment) jobs sorted by
+// address, cut into tiles of up to 32 jobs whose segments fit a window of 32 ksteps positions, the
+// window with the fewest k-steps in all.  Returns false (no tiles set) where the VALU gathers are
+// the faster form.
+bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
+                                    const std::vector<uint16_t> &wraw,
+                                    const std::vector<uint64_t> &starts) {
+    const int force = tune(Tune::Jobs);
+    if (force == 0 || tune(Tune::Path) == 0 || wx.S < 32u || wx.step % 8u != 0u) return false;
+    // switches that pick a form of the VALU gathers keep them
+    for (Tune t : {Tune::Lane8, Tune::KSplit, Tune::StreamKernel, Tune::WeightsInLds,
+                   Tune::NonTemporal, Tune::SortSegments})
+        if (force < 0 && tune(t) >= 0) return false;
+    const uint64_t n_jobs = (uint64_t)c.Cout * wx.K;
+    // sums: 32-bit rows, at most 256 MiB of scratch
+    if (n_jobs * wx.tokens * 4u > (256ull << 20)) return false;
+    const uint64_t lo = *std::min_element(starts.begin(), starts.end());
+    const uint64_t hi = *std::max_element(starts.begin(), starts.end());
+    if (hi - lo + (uint64_t)wx.S * wx.step > 0xffffffffull) return false;
+    for (uint64_t s : starts)
+        if (s % 8u != 0u || (s - lo) % wx.step != 0u) return false;
+    if (wx.tokens % 64u != 0u || wx.out_stride % 4u != 0u || wx.y_off % 4u != 0u ||
+        (wx.has_res && wx.res_off % 4u != 0u))
+        return false;
+    // (position, job) in address order
+    std::vector<uint64_t> jobs(n_jobs);
+    for (uint64_t j = 0; j < c.Cout; ++j)
+        for (uint64_t k = 0; k < wx.K; ++k)
+            jobs[j * wx.K + k] =
+                (starts[j / c.cluster_size * wx.K + k] - lo) / wx.step << 32 | (j * wx.K + k);
+    std::sort(jobs.begin(), jobs.end());
+    constexpr uint32_t slots = 16u * k44dev::K44_JOB_BLOCKS;
+    auto cut = [&](uint32_t ks, std::vector<uint32_t> *first) {
+        uint64_t tiles = 0, base = 0;
+        uint32_t fill = 0;
+        for (uint64_t i = 0; i < n_jobs; ++i) {
+            const uint64_t p = jobs[i] >> 32;
+            if (fill == 0u || fill == slots || p + wx.S > base + 32u * ks) {
+                if (first) first->push_back((uint32_t)i);
+                ++tiles;
+                base = p;
+                fill = 0;
+            }
+            ++fill;
+        }
+        return tiles;
+    };
+    uint64_t best = UINT64_MAX;  // k-steps of all tiles
+    for (uint32_t e = 0; e < 3u; ++e) {
+        const uint32_t ks = (wx.S + 31u) / 32u + e;
+        const uint64_t steps = cut(ks, nullptr) * ks;
+        if (steps >= best) continue;
+        best = steps;
+        wx.jb_ksteps = ks;
+    }
+    // Times in us that fit both forms over 96 to 8,192 neurons of 2 to 16 segments of 32 to 512
+    // positions over 16 to 256 tokens.  Job tiles: 0.35 ns per tile's k-step and 64 tokens, the
+    // sums at 5 TB/s, the chain of gathers.  The VALU gathers: their bytes at 22 TB/s from L2, 9
+    // once the rows exceed it, or a neuron's chain of rows.  (8,192 x 2 x 32 over 256 tokens: 15.1
+    // us gathered, 16.1 as jobs, 512 x 4 x 32 over 16 tokens 4.9 and 7.3; 512 x 8 x 128 over 64
+    // tokens 15.9 and 7.7, 4,096 x 8 x 64 over 32 tokens 16.0 and 11.0.)
+    const double t64 = wx.tokens / 64u;
+    const double mb = (double)n_jobs * wx.tokens * 1e-6, x_mb = (double)(hi - lo) * 2e-6;
+    const double t_jobs = 6.0 + 0.25 * wx.jb_ksteps + 0.00035 * (double)best * t64 + 1.6 * mb;
+    const double t_valu = std::max(2.0 + 0.0135 * wx.K * wx.S,
+                                   4.0 + 2.0 * mb * wx.S / (x_mb <= 32.0 ? 22.0 : 9.0));
+    if (force < 0 && t_jobs >= 0.85 * t_valu) return false;
+    std::vector<uint32_t> first;
+    wx.jb_tiles = (uint32_t)cut(wx.jb_ksteps, &first);
+    first.push_back((uint32_t)n_jobs);
+    const uint32_t per = 32u * wx.jb_ksteps;
+    std::vector<uint32_t> ro((size_t)wx.jb_tiles * per), jm((size_t)wx.jb_tiles * slots, 0xffffffffu),
+        ko(jm.size(), 0u);
+    std::vector<uint16_t> wf((size_t)wx.jb_tiles * per * slots, 0u);
+    for (size_t t = 0; t < wx.jb_tiles; ++t) {
+        const uint64_t base = jobs[first[t]] >> 32;
+        uint32_t *rt = &ro[t * per];
+        std::fill(rt, rt + per, (uint32_t)(base * wx.step));  // rows no job reads: the first one
+        uint32_t done = 0;  // window rows set so far (jobs are in address order)
+        for (uint32_t i = first[t]; i < first[t + 1]; ++i) {
+            const uint32_t n = i - first[t], id = (uint32_t)jobs[i];
+            const uint32_t off = (uint32_t)((jobs[i] >> 32) - base);
+            for (done = std::max(done, off); done < off + wx.S; ++done)
+                rt[done] = (uint32_t)((base + done) * wx.step);
+            jm[t * slots + n] = id;
+            ko[t * slots + n] = off;
+            const uint16_t *src = &wraw[(size_t)(id / wx.K) * c.B + (size_t)(id % wx.K) * wx.S];
+            uint16_t *dst = &wf[t * per * slots + ((n >> 4) * 64u + (n & 15u)) * 8u];
+            for (uint32_t p = off; p < off + wx.S; ++p)
+                dst[((p >> 5) * k44dev::K44_JOB_BLOCKS * 64u + ((p & 31u) >> 3) * 16u) * 8u + (p & 7u)] = src[p - off];
+        }
+    }
+    wx.rk_base = lo;
+    wx.roff.upload(ro);
+    wx.jmap.upload(jm);
+    wx.koff.upload(ko);
+    wx.w.alloc(wf.size());
+    K44_HIP(hipMemcpy(wx.w.p, wf.data(), wf.size() * 2u, hipMemcpyHostToDevice));
+    wx.part_floats = (size_t)n_jobs * wx.tokens;
+    wx.why += "; segments as MFMA jobs: " + std::to_string(wx.jb_tiles) + " tiles of " +
+              std::to_string(slots) + " over windows of " + std::to_string(per) + " positions";
+    return true;
+}
+
 // Waves per tile: 8 (4 for short rows) while there is at most a tile of 64 tokens per CU (64 x 4
 // tiles of 512 scattered inputs 6.1 us, 6.8 with 4; 64 x 8 tiles of 8,192 inputs, rows from HBM,
 // 110 us, 88 with 4; of 600 scattered inputs 11.1 and 10.7), then 4, and 1 once the tiles alone
@@ -568,21 +672,24 @@ void K44GpuExecutorState::build_wave(const K44ExecCmd &c, WaveExec &wx) {
                           "staged in LDS";
             }
         }
+        if (!wx.stream_kernel && !wx.misaligned) job_tiles(c, wx, wraw, starts);
         const uint32_t rpi = 256u / wx.slab;
         wx.U = 16u / rpi;
         const uint32_t per_batch = rpi * wx.U;
         wx.n_batch = (wx.S + per_batch - 1u) / per_batch;
-        std::vector<uint16_t> wk((size_t)c.Cout * wx.K * wx.n_batch * per_batch, 0u);
-        for (size_t j = 0; j < c.Cout; ++j)
+        std::vector<uint16_t> wk(wx.jb_tiles ? 0u : (size_t)c.Cout * wx.K * wx.n_batch * per_batch, 0u);
+        for (size_t j = 0; j < c.Cout && !wx.jb_tiles; ++j)
             for (uint32_t k = 0; k < wx.K; ++k)
                 for (uint32_t s = 0; s < wx.S; ++s) {
                     const uint32_t b = s / per_batch, q = s % per_batch;  // q = g*U + u
                     wk[((j * wx.K + k) * wx.n_batch + b) * per_batch + q] =
                         wraw[j * c.B + (size_t)k * wx.S + s];
                 }
-        std::vector<__half> wh(wk.size());
-        std::memcpy(wh.data(), wk.data(), wk.size() * 2u);
-        wx.w.upload(wh);
+        if (!wx.jb_tiles) {
+            std::vector<__half> wh(wk.size());
+            std::memcpy(wh.data(), wk.data(), wk.size() * 2u);
+            wx.w.upload(wh);
+        }
     }
     if (wx.narrow) wx.seg_h = starts;
     wx.seg.upload(starts);

@@ -106,6 +106,34 @@ void K44GpuExecutorState::launch_mfma_group(const k44dev::MfmaGroup &d, uint32_t
     if (epi_items) K44_HIP(k44dev::launch_splitk_epilogue(d, epi_items, stream));
 }
 
+void K44GpuExecutorState::launch_jobs(const WaveExec &w) {
+    k44dev::JobArgs a{};
+    a.X = canvas.p + w.rk_base;
+    a.roff = w.roff.p;
+    a.Wf = w.w.p;
+    a.jmap = w.jmap.p;
+    a.koff = w.koff.p;
+    a.part = scratch.p;
+    a.ksteps = w.jb_ksteps;
+    a.tiles = w.jb_tiles;
+    a.ttiles = w.tokens / 64u;
+    a.tokens = w.tokens;
+    a.S = w.S;
+    K44_HIP(k44dev::launch_mfma_jobs(a, stream));
+    k44dev::JobReduceArgs r{};
+    r.part = scratch.p;
+    r.bias = w.bias.p;
+    r.cmap = w.cmap.p;
+    r.Y = canvas.p + w.y_off;
+    r.R = w.has_res ? canvas.p + w.res_off : nullptr;
+    r.out_stride = w.out_stride;
+    r.cout = w.cout;
+    r.K = w.K;
+    r.tokens = w.tokens;
+    r.act = w.act;
+    K44_HIP(k44dev::launch_jobs_reduce(r, stream));
+}
+
 k44dev::RowsArgs K44GpuExecutorState::rows_args(const WaveExec &w, bool fused) const {
     k44dev::RowsArgs a{};
     a.X = canvas.p + w.rk_base;
@@ -169,6 +197,10 @@ void K44GpuExecutorState::launch_group(const MfmaGroupExec &g) {
 }
 
 void K44GpuExecutorState::launch_wave(const WaveExec &w) {
+    if (w.jb_tiles) {
+        launch_jobs(w);
+        return;
+    }
     if (w.rowsk) {
         launch_rows(w);
         if (w.tile2d)

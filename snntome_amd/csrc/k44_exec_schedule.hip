@@ -1239,7 +1239,7 @@ size_t K44GpuExecutorState::launches_per_run() const {
         if (r.first == 2) n += groups[r.second]->epi_items ? 2u : 1u;
         else if (r.first == 0 && aux[r.second]->type == K44CmdType::ARGMAX_1D)
             n += hist_steps ? 3u : 2u;
-        else n += 1u;
+        else n += r.first == 1 && waves[r.second]->jb_tiles ? 2u : 1u;
     }
     return n;
 }
@@ -1255,7 +1255,7 @@ void K44GpuExecutorState::build_report() {
           << ", \"tokens\": " << w.tokens << ", \"slab\": " << (w.mfma ? w.mt : w.slab)
           << ", \"U\": " << (w.mfma ? w.rows_per_stage : w.U)
           << ", \"ksplit\": " << (w.rowsk ? w.rk_kw : w.mfma ? w.kgroups : w.ksplit)
-          << ", \"kernel\": \"" << (w.rowsk ? "rows" : w.path.substr(w.path.find('_') + 1u)) << "\""
+          << ", \"kernel\": \"" << (w.rowsk ? "rows" : w.jb_tiles ? "jobs" : w.path.substr(w.path.find('_') + 1u)) << "\""
           << ", \"sorted_segments\": " << (w.sorted_segments ? "true" : "false")
           << ", \"misaligned\": " << (w.misaligned ? "true" : "false")
           << ", \"phase_order\": " << (w.phase_order ? "true" : "false")

@@ -30,6 +30,7 @@
 #include "k44wavec.h"
 #include "kernels/k44_hostio.hpp"
 #include "kernels/k44_launch.hpp"
+#include "kernels/k44_mfma_jobs.hpp"
 #include "kernels/k44_mfma_rows.hpp"
 #include "kernels/k44_program.hpp"
 #include "kernels/k44_spatial.hpp"
@@ -181,6 +182,10 @@ struct WaveExec {
     DevBuf<uint32_t> roff;
     uint32_t rk_ttiles() const { return tokens / 64u; }
     uint64_t rk_tiles() const { return (uint64_t)rows * rk_subs * rk_ttiles(); }
+    // Segments of private index rows as MFMA jobs (k44_mfma_jobs.hip): tiles (0: not used), their
+    // window's k-steps, tables; sums in the plan's scratch.
+    uint32_t jb_tiles = 0, jb_ksteps = 0;
+    DevBuf<uint32_t> jmap, koff;
     // 2-D spatial wave (VALU over the padded-plane tile layout): tile tables, output plane.
     bool tile2d = false;
     DevBuf<uint32_t> tile_x, tile_y;
@@ -390,6 +395,8 @@ struct K44GpuExecutorState {
                         size_t rows, uint32_t width);
     bool rows_shape(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint64_t> &starts,
                     const std::vector<uint32_t> &tx, const std::vector<uint32_t> &ty);
+    bool job_tiles(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
+                   const std::vector<uint64_t> &starts);
     static uint32_t rows_waves(uint64_t tiles, uint32_t ksteps);
     static void use_rows(WaveExec &wx, uint32_t kw);
     k44dev::RowsArgs rows_args(const WaveExec &w, bool fused) const;
@@ -440,6 +447,7 @@ struct K44GpuExecutorState {
                            uint32_t prod, uint32_t max_items, bool mis,
                            const k44dev::NarrowPre &pre);
     void launch_rows(const WaveExec &w);
+    void launch_jobs(const WaveExec &w);
     void launch_mfma(const WaveExec &w);
     void launch_group(const MfmaGroupExec &g);
     void launch_wave(const WaveExec &w);

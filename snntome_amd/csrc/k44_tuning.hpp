@@ -55,6 +55,8 @@ enum class Tune : int {
     NarrowByy,     // "narrow_byy":    0 = narrow group launches find each workgroup's wave in the
                    //                  group's prefix sums; automatic: (workgroups x waves) grids
                    //                  where they launch at most 1.5x the work items
+    Jobs,          // "jobs":          0 = no MFMA job tiles for private segments, 1 = wherever
+                   //                  they apply
     Rows,          // "rows":          0 = no row-table MFMA kernel, 1 | 4 | 8 = waves per tile in it
     Count
 };
