@@ -200,6 +200,9 @@ __global__ __launch_bounds__(64 * (KW == 1 ? 4 : KW)) void k44_mfma_rows_kernel(
             load_a(min(ks + KW, a.ksteps - 1u));
             load_x(rn);
             rn = roff[(uint64_t)min(ks + 2u * KW, a.ksteps - 1u) * 8u];
+            // KW = 1: or the compiler sinks these loads to their use (a dense block over 4,096 tokens
+            // 273 us, 258 so; with more waves per tile it costs up to 3 %)
+            if constexpr (KW == 1) asm volatile("" ::: "memory");
 #pragma unroll
             for (int tb = 0; tb < 4; ++tb) {
                 const _Float16 *p = &xs[tr_row][tr_col + 16 * tb];
