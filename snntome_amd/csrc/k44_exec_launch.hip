@@ -166,6 +166,11 @@ k44dev::RowsArgs K44GpuExecutorState::rows_args(const WaveExec &w, bool fused) c
 void K44GpuExecutorState::launch_rows(const WaveExec &w) {
     k44dev::RowsLaunch l;
     l.one = rows_args(w, false);
+    if (w.tile2d && !w.plane.tok64 && w.rk_mis) {
+        l.halo = canvas.p + w.y_off;
+        l.halo_planes = w.cout * w.plane.frames;
+        l.plane = w.plane;
+    }
     K44_HIP(k44dev::launch_mfma_rows(l, w.rows * w.rk_subs, w.rk_ttiles(), w.rk_nb, w.rk_kw,
                                      w.rk_mis, stream));
 }
@@ -203,7 +208,7 @@ void K44GpuExecutorState::launch_wave(const WaveExec &w) {
     }
     if (w.rowsk) {
         launch_rows(w);
-        if (w.tile2d)
+        if (w.tile2d && (w.plane.tok64 || !w.rk_mis))
             K44_HIP(k44dev::launch_halo_clear(canvas.p + w.y_off, w.cout, w.plane, stream));
         return;
     }

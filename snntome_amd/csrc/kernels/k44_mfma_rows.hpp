@@ -1,6 +1,7 @@
 // k44_mfma_rows.hpp — MFMA waves whose tiles gather arbitrary rows (see k44_mfma_rows.hip).
 #pragma once
 #include "k44_mfma_tile.hpp"
+#include "k44_spatial.hpp"
 
 namespace k44dev {
 
@@ -38,6 +39,11 @@ struct RowsLaunch {
     uint32_t n = 0;
     uint32_t by_cols = 0;  // token tiles when items are numbered column by column (launcher)
     RowsArgs one{};
+    // 2-D waves (mis kernels only; not interleaved frames): the zero frame of the output planes,
+    // cleared by a second layer of workgroups (blockIdx.z = 1), or nullptr.
+    __half *halo = nullptr;
+    uint32_t halo_planes = 0;
+    Plane2D plane{};
 };
 
 // cols: workgroup columns (index rows x sub-tiles, all waves); ttiles: the most 64-token tiles of

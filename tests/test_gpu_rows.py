@@ -166,3 +166,33 @@ def test_long_rows_keep_their_split(wavec):
         kernels[tokens] = plan.exec_report()["waves"][0]["kernel"]
         plan.release_gpu()
     assert kernels == {64: "tile", 320: "rows"}
+
+
+@pytest.mark.parametrize("frames,H,W,cin,cout,kw", [
+    (1, 5, 128, 8, 16, 1), (3, 7, 21, 24, 48, 4), (1, 3, 5, 16, 16, 8), (2, 40, 50, 3, 32, -1),
+])
+def test_halos_are_cleared(wavec, tuning, frames, H, W, cin, cout, kw):
+    """Whatever the output planes held, all but the image pixels is zero after the convolution,
+    and a second run gives the same bits."""
+    rng = np.random.default_rng(W)
+    tuning("rows", kw)
+    w = rng.standard_normal((cout, cin, 3, 3)).astype(np.float32)
+    g = wavec.WaveGraph(kv_cache_max_seq=0, batch_size=frames)
+    g.add_input("img", cin, H, W)
+    g.add_conv2d("c", "img", "y", cin, cout, 3, 3, w, np.ones(cout, np.float32), stride=1, pad=1)
+    plan = g.compile()
+    plan.init_gpu()
+    lay = co.Layout2D(H, W, frames)
+    x = np.zeros(cin * lay.channel_stride, np.float16)
+    x[lay.offsets(cin).ravel()] = rng.standard_normal(frames * cin * H * W).astype(np.float16)
+    plan.write_canvas(int(plan.cmds[0]["src_off"]), x)
+    plan.execute(1)
+    y0, n = int(plan.cmds[0]["y_off"]), cout * lay.channel_stride
+    first = plan.read_canvas(y0, n)
+    plan.write_canvas(y0, np.full(n, 0x3c00, np.uint16))
+    plan.execute(1)
+    out = plan.read_canvas(y0, n)
+    halo = np.ones(n, bool)
+    halo[lay.offsets(cout).ravel()] = False
+    assert not out[halo].any() and first[~halo].any()
+    assert np.array_equal(out, first)
