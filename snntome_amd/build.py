@@ -34,7 +34,8 @@ SOURCES = ["k44_wave_executor.hip", "k44_exec_build.hip", "k44_exec_schedule.hip
            "kernels/k44_mfma_nt16.hip", "kernels/k44_mfma_nt32.hip", "kernels/k44_mfma_nt64.hip",
            "kernels/k44_mfma_nt128.hip", "kernels/k44_mfma_narrow.hip", "kernels/k44_mfma_dma.hip", "kernels/k44_token64.hip",
            "kernels/k44_spatial.hip", "kernels/k44_program.hip", "kernels/k44_hostio.hip",
-           "kernels/k44_mfma_rows.hip", "kernels/k44_mfma_jobs.hip"]
+           "kernels/k44_mfma_rows.hip", "kernels/k44_mfma_jobs.hip",
+           "kernels/k44_row_list.hip"]
 BUILD_DIR = HERE / "_build"
 
 

@@ -402,6 +402,53 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
     return true;
 }
 
+// Offset lists of a wave with segments under 32 positions, of 16 and more (the segment gathers'
+// batch) only while the rows of a token tile take at most two XCDs' L2: 4,096 x 8 x 16 of 65,536
+// rows over 256 tokens 33.1 us as segments, 28.7 as lists, 1,024 x 8 x 24 of 20,000 over 64 7.2 and
+// 5.0, but 8,192 x 12 x 16 of 131,072 over 64 20.5 and 25.4.
+// Returns false (nothing set) for those, for rows off the 16-byte grid or beyond 32-bit offsets.
+bool K44GpuExecutorState::row_list(const K44ExecCmd &c, WaveExec &wx,
+                                   const std::vector<uint16_t> &wraw,
+                                   const std::vector<uint64_t> &starts) {
+    if (wx.S >= 32u || (wx.S >= 16u && wx.unique_rows * 128u > (8ull << 20)) ||
+        tune(Tune::Rows) == 0 || wx.tokens % 64u != 0u || wx.step % 8u != 0u ||
+        wx.out_stride % 8u != 0u || wx.y_off % 8u != 0u || (wx.has_res && wx.res_off % 8u != 0u))
+        return false;
+    // switches that pick a form of the segment gathers keep them
+    for (Tune t : {Tune::Lane8, Tune::KSplit, Tune::StreamKernel, Tune::WeightsInLds,
+                   Tune::NonTemporal, Tune::SortSegments})
+        if (tune(t) >= 0) return false;
+    const uint64_t lo = *std::min_element(starts.begin(), starts.end());
+    const uint64_t hi = *std::max_element(starts.begin(), starts.end());
+    if (hi - lo + (uint64_t)wx.S * wx.step > 0xffffffffull || wx.tokens / 64u > 65535u) return false;
+    for (uint64_t s : starts)
+        if (s % 8u != 0u) return false;
+    const uint32_t fan = wx.K * wx.S, per = (fan + 31u) / 32u * 32u;
+    std::vector<uint32_t> ro((size_t)wx.rows * per);
+    for (size_t r = 0; r < wx.rows; ++r) {
+        uint32_t *q = &ro[r * per];
+        for (uint32_t k = 0; k < wx.K; ++k)
+            for (uint32_t s = 0; s < wx.S; ++s)
+                q[k * wx.S + s] = (uint32_t)(starts[r * wx.K + k] + (uint64_t)s * wx.step - lo);
+        std::fill(q + fan, q + per, q[fan - 1u]);
+    }
+    std::vector<__half> w((size_t)c.Cout * per);
+    for (size_t j = 0; j < c.Cout; ++j) {
+        std::memset((void *)&w[j * per], 0, per * 2u);
+        std::memcpy((void *)&w[j * per], &wraw[j * c.B], fan * 2u);
+    }
+    wx.rk_base = lo;
+    wx.roff.upload(ro);
+    wx.w.upload(w);
+    // Four waves per neuron while one would leave the chip at most 2 per CU and each has some steps
+    // (256 x 250 over 10 tokens 3.9 us, 5.3 with one; 1,024 x 100 over 64 4.7 and 4.4).
+    wx.rl_kw = (uint64_t)c.Cout * (wx.tokens / 64u) <= 512u && per >= 128u ? 4u : 1u;
+    if (tune(Tune::Rows) > 0) wx.rl_kw = tune(Tune::Rows) == 1 ? 1u : 4u;
+    wx.ksplit = wx.rl_kw;
+    wx.why += "; lists of row offsets, " + std::to_string(wx.rl_kw) + " waves per neuron";
+    return true;
+}
+
 // Waves per tile: 8 (4 for short rows) while there is at most a tile of 64 tokens per CU (64 x 4
 // tiles of 512 scattered inputs 6.1 us, 6.8 with 4; 64 x 8 tiles of 8,192 inputs, rows from HBM,
 // 110 us, 88 with 4; of 600 scattered inputs 11.1 and 10.7), then 4, and 1 once the tiles alone
@@ -672,20 +719,22 @@ void K44GpuExecutorState::build_wave(const K44ExecCmd &c, WaveExec &wx) {
                           "staged in LDS";
             }
         }
-        if (!wx.stream_kernel && !wx.misaligned) job_tiles(c, wx, wraw, starts);
+        if (!wx.stream_kernel && !wx.misaligned && !job_tiles(c, wx, wraw, starts))
+            row_list(c, wx, wraw, starts);
+        const bool own_weights = wx.jb_tiles || wx.rl_kw;
         const uint32_t rpi = 256u / wx.slab;
         wx.U = 16u / rpi;
         const uint32_t per_batch = rpi * wx.U;
         wx.n_batch = (wx.S + per_batch - 1u) / per_batch;
-        std::vector<uint16_t> wk(wx.jb_tiles ? 0u : (size_t)c.Cout * wx.K * wx.n_batch * per_batch, 0u);
-        for (size_t j = 0; j < c.Cout && !wx.jb_tiles; ++j)
+        std::vector<uint16_t> wk(own_weights ? 0u : (size_t)c.Cout * wx.K * wx.n_batch * per_batch, 0u);
+        for (size_t j = 0; j < c.Cout && !own_weights; ++j)
             for (uint32_t k = 0; k < wx.K; ++k)
                 for (uint32_t s = 0; s < wx.S; ++s) {
                     const uint32_t b = s / per_batch, q = s % per_batch;  // q = g*U + u
                     wk[((j * wx.K + k) * wx.n_batch + b) * per_batch + q] =
                         wraw[j * c.B + (size_t)k * wx.S + s];
                 }
-        if (!wx.jb_tiles) {
+        if (!own_weights) {
             std::vector<__half> wh(wk.size());
             std::memcpy(wh.data(), wk.data(), wk.size() * 2u);
             wx.w.upload(wh);

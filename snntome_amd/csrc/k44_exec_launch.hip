@@ -134,6 +134,25 @@ void K44GpuExecutorState::launch_jobs(const WaveExec &w) {
     K44_HIP(k44dev::launch_jobs_reduce(r, stream));
 }
 
+void K44GpuExecutorState::launch_list(const WaveExec &w) {
+    k44dev::RowListArgs a{};
+    a.X = canvas.p + w.rk_base;
+    a.roff = w.roff.p;
+    a.W = w.w.p;
+    a.bias = w.bias.p;
+    a.cmap = w.cmap.p;
+    a.Y = canvas.p + w.y_off;
+    a.R = w.has_res ? canvas.p + w.res_off : nullptr;
+    a.out_stride = w.out_stride;
+    a.cout = w.cout;
+    a.cluster = w.cluster;
+    a.B = w.K * w.S;
+    a.steps = (a.B + 31u) / 32u;
+    a.ttiles = w.tokens / 64u;
+    a.act = w.act;
+    K44_HIP(k44dev::launch_row_list(a, w.rl_kw, stream));
+}
+
 k44dev::RowsArgs K44GpuExecutorState::rows_args(const WaveExec &w, bool fused) const {
     k44dev::RowsArgs a{};
     a.X = canvas.p + w.rk_base;
@@ -204,6 +223,10 @@ void K44GpuExecutorState::launch_group(const MfmaGroupExec &g) {
 void K44GpuExecutorState::launch_wave(const WaveExec &w) {
     if (w.jb_tiles) {
         launch_jobs(w);
+        return;
+    }
+    if (w.rl_kw) {
+        launch_list(w);
         return;
     }
     if (w.rowsk) {

@@ -1255,7 +1255,7 @@ void K44GpuExecutorState::build_report() {
           << ", \"tokens\": " << w.tokens << ", \"slab\": " << (w.mfma ? w.mt : w.slab)
           << ", \"U\": " << (w.mfma ? w.rows_per_stage : w.U)
           << ", \"ksplit\": " << (w.rowsk ? w.rk_kw : w.mfma ? w.kgroups : w.ksplit)
-          << ", \"kernel\": \"" << (w.rowsk ? "rows" : w.jb_tiles ? "jobs" : w.path.substr(w.path.find('_') + 1u)) << "\""
+          << ", \"kernel\": \"" << (w.rowsk ? "rows" : w.jb_tiles ? "jobs" : w.rl_kw ? "row_list" : w.path.substr(w.path.find('_') + 1u)) << "\""
           << ", \"sorted_segments\": " << (w.sorted_segments ? "true" : "false")
           << ", \"misaligned\": " << (w.misaligned ? "true" : "false")
           << ", \"phase_order\": " << (w.phase_order ? "true" : "false")

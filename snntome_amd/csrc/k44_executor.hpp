@@ -33,6 +33,7 @@
 #include "kernels/k44_mfma_jobs.hpp"
 #include "kernels/k44_mfma_rows.hpp"
 #include "kernels/k44_program.hpp"
+#include "kernels/k44_row_list.hpp"
 #include "kernels/k44_spatial.hpp"
 
 namespace k44_host {
@@ -186,6 +187,8 @@ struct WaveExec {
     // window's k-steps, tables; sums in the plan's scratch.
     uint32_t jb_tiles = 0, jb_ksteps = 0;
     DevBuf<uint32_t> jmap, koff;
+    // Scattered private index rows as offset lists (k44_row_list.hip): waves per neuron (0: not used).
+    uint32_t rl_kw = 0;
     // 2-D spatial wave (VALU over the padded-plane tile layout): tile tables, output plane.
     bool tile2d = false;
     DevBuf<uint32_t> tile_x, tile_y;
@@ -397,6 +400,8 @@ struct K44GpuExecutorState {
                     const std::vector<uint32_t> &tx, const std::vector<uint32_t> &ty);
     bool job_tiles(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
                    const std::vector<uint64_t> &starts);
+    bool row_list(const K44ExecCmd &c, WaveExec &wx, const std::vector<uint16_t> &wraw,
+                  const std::vector<uint64_t> &starts);
     static uint32_t rows_waves(uint64_t tiles, uint32_t ksteps);
     static void use_rows(WaveExec &wx, uint32_t kw);
     k44dev::RowsArgs rows_args(const WaveExec &w, bool fused) const;
@@ -448,6 +453,7 @@ struct K44GpuExecutorState {
                            const k44dev::NarrowPre &pre);
     void launch_rows(const WaveExec &w);
     void launch_jobs(const WaveExec &w);
+    void launch_list(const WaveExec &w);
     void launch_mfma(const WaveExec &w);
     void launch_group(const MfmaGroupExec &g);
     void launch_wave(const WaveExec &w);

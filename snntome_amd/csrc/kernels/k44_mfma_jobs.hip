@@ -10,7 +10,7 @@
 // the matrix cores.  Every job's fp32 sums go to a row of their own, and a second kernel adds a
 // neuron's K rows in segment order and runs the epilogue (34 MB written and read).
 // That wave: 87 us as gathers, 25 as job tiles; 8,192 x 12 x 128 over 256 tokens of 130,000 rows
-// 769 and 58; 2,048 x 16 x 128 over 64 tokens 19.1 and 12.1.  Tiles of 64 jobs, with half the
+// 769 and 58; 4,096 x 8 x 64 over 64 tokens 19.1 and 12.1.  Tiles of 64 jobs, with half the
 // windows but twice the zero products, were never faster (31, 61 and 12.5 us).
 // Bound now by the gather's latency (a k-step's rows come one step ahead) and the sums' traffic.
 //
