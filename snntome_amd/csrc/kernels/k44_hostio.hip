@@ -7,6 +7,8 @@
 // 32 x 160 x 160 input (819 k in, 410 k out) 1952 -> 472 us.
 #include "k44_hostio.hpp"
 
+#include "k44_pack_index.hpp"
+
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -152,8 +154,9 @@ __global__ __launch_bounds__(256) void k44_pack_rows_kernel(uint16_t *dst, const
                                                             I first, I n, uint64_t row_stride,
                                                             I cols) {
     for (I q = ((I)blockIdx.x * 256u + threadIdx.x) * 8u; q < n; q += (I)gridDim.x * 2048u) {
-        I r = (first + q) / cols, c = first + q - r * cols;
-        const uint16_t *p = src + (uint64_t)r * row_stride;
+        RowCol<I> at = row_col<I>(first + q, cols);
+        I &c = at.c;
+        const uint16_t *p = src + (uint64_t)at.r * row_stride;
         if constexpr (VEC) {
             *reinterpret_cast<us8 *>(dst + q) = *reinterpret_cast<const us8 *>(p + c);
         } else {
@@ -181,12 +184,10 @@ template <bool VEC>
 static void pack_rows(uint16_t *dst, const uint16_t *src, uint64_t first, uint64_t n,
                       uint64_t row_stride, uint64_t cols, hipStream_t stream) {
     const dim3 grid((uint32_t)std::min<uint64_t>((n + 2047u) / 2048u, 2048u));
-    if (first + n < (1ull << 31))  // (32-bit division; the loop's last step stays below 2^32)
-        hipLaunchKernelGGL((k44_pack_rows_kernel<VEC, uint32_t>), grid, dim3(256), 0, stream, dst,
-                           src, (uint32_t)first, (uint32_t)n, row_stride, (uint32_t)cols);
-    else
-        hipLaunchKernelGGL((k44_pack_rows_kernel<VEC, uint64_t>), grid, dim3(256), 0, stream, dst,
-                           src, first, n, row_stride, cols);
+    with_pack_index(first, n, cols, [&](auto f, auto k, auto w) {
+        hipLaunchKernelGGL((k44_pack_rows_kernel<VEC, decltype(f)>), grid, dim3(256), 0, stream, dst,
+                           src, f, k, row_stride, w);
+    });
 }
 
 hipError_t launch_pack_rows(uint16_t *dst, const uint16_t *src, uint64_t first, uint64_t n,
