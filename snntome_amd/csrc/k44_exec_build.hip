@@ -353,6 +353,14 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
         best = steps;
         wx.jb_ksteps = ks;
     }
+    // Fragments, zero-padded to 32 jobs per window: at most 3 times the weights, or 32 MiB (all
+    // L2s) where jobs are too far apart for that.  Beyond, memory and set-up grow without bound (a
+    // job per tile holds 32 times its weights) and the time goes with them: 4,096 x 16 x 128 over
+    // 64 tokens of 4 M positions 390 MB of fragments, 179 us, 145 gathered; 4,096 x 8 x 64 of 1 M
+    // 86 MB, 40 and 40; 2,048 x 4 x 256 over 128 tokens of 1 M 109 MB, 74 and 75.  (Some would still
+    // gain, as 4,096 x 16 x 512 over 64 tokens of 1 M positions: 172 and 513 for 7 times the weights.)
+    const uint64_t frag = best * k44dev::K44_JOB_BLOCKS * 1024u;
+    if (frag > std::max<uint64_t>(32ull << 20, 3u * n_jobs * wx.S * 2u)) return false;
     // Times in us that fit both forms over 96 to 8,192 neurons of 2 to 16 segments of 32 to 512
     // positions over 16 to 256 tokens.  Job tiles: 0.35 ns per tile's k-step and 64 tokens, the
     // sums at 5 TB/s, the chain of gathers.  The VALU gathers: their bytes at 22 TB/s from L2, 9
@@ -361,9 +369,13 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
     // tokens 15.9 and 7.7, 4,096 x 8 x 64 over 32 tokens 16.0 and 11.0.)
     const double t64 = wx.tokens / 64u;
     const double mb = (double)n_jobs * wx.tokens * 1e-6, x_mb = (double)(hi - lo) * 2e-6;
-    const double t_jobs = 6.0 + 0.25 * wx.jb_ksteps + 0.00035 * (double)best * t64 + 1.6 * mb;
-    const double t_valu = std::max(2.0 + 0.0135 * wx.K * wx.S,
-                                   4.0 + 2.0 * mb * wx.S / (x_mb <= 32.0 ? 22.0 : 9.0));
+    double t_jobs = 6.0 + 0.25 * wx.jb_ksteps + 0.00035 * (double)best * t64 + 1.6 * mb;
+    double t_valu = std::max(2.0 + 0.0135 * wx.K * wx.S,
+                             4.0 + 2.0 * mb * wx.S / (x_mb <= 32.0 ? 22.0 : 9.0));
+    // Beyond the 256 MB MALL everything that a form reads once comes from HBM, at 6.5 TB/s.
+    const double rows_mb = (double)wx.unique_rows * wx.tokens * 2e-6, all_mb = rows_mb + (double)frag * 1e-6;
+    if (all_mb > 256.0) t_jobs = std::max(t_jobs, all_mb / 6.5);
+    if (rows_mb > 256.0) t_valu = std::max(t_valu, rows_mb / 6.5);
     if (force < 0 && t_jobs >= 0.85 * t_valu) return false;
     std::vector<uint32_t> first;
     wx.jb_tiles = (uint32_t)cut(wx.jb_ksteps, &first);

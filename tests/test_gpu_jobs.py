@@ -67,3 +67,22 @@ def test_unread_infinities_stay_out(wavec, tuning):
     xh = np.where(np.isfinite(x), x, 0).astype(np.float16).astype(np.float64)[:, 0, :]
     ref = np.einsum("js,jst->jt", w.astype(np.float64), xh[syn])
     assert np.abs(rest - np.delete(ref, [3, 69], axis=1)).max() <= 2.0 ** -10 * ref.max()
+
+
+@pytest.mark.parametrize("C,cout,K,S,tokens,kernel", [
+    (65536, 4096, 8, 64, 64, "jobs"),            # segments overlap 32 times
+    (200_000, 512, 8, 128, 64, "jobs"),          # few jobs per window, 11 MiB of fragments
+    (1 << 20, 2048, 4, 256, 128, "gather_dot"),  # 109 MB of fragments for 4 MB of weights
+    (1 << 20, 4096, 8, 64, 64, "gather_dot"),    # 86 MB for 4
+])
+def test_automatic_choice(wavec, tuning, C, cout, K, S, tokens, kernel):
+    """Job tiles where segments overlap; not where their padded fragments would grow without bound."""
+    rng = np.random.default_rng(S)
+    starts = (rng.integers(0, (C - S) // 8 + 1, (cout, K)) * 8).astype(np.uint32)
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", C, 1, tokens, is_1d=True)
+    g.add_cluster_wave("w", "x", "y", starts, S, np.ones((cout, K * S), np.float16), None, cluster=1)
+    plan = g.compile()
+    plan.init_gpu()
+    assert plan.exec_report()["waves"][0]["kernel"] == kernel
+    plan.release_gpu()
