@@ -319,6 +319,8 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
     if (hi - lo + (uint64_t)wx.S * wx.step > 0xffffffffull) return false;
     for (uint64_t s : starts)
         if (s % 8u != 0u || (s - lo) % wx.step != 0u) return false;
+    for (uint16_t v : wraw)  // (the kernel's second pass over non-finite rows counts on it)
+        if ((v & 0x7c00u) == 0x7c00u) return false;
     if (wx.tokens % 64u != 0u || wx.out_stride % 4u != 0u || wx.y_off % 4u != 0u ||
         (wx.has_res && wx.res_off % 4u != 0u))
         return false;

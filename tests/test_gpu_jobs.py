@@ -69,6 +69,56 @@ def test_unread_infinities_stay_out(wavec, tuning):
     assert np.abs(rest - np.delete(ref, [3, 69], axis=1)).max() <= 2.0 ** -10 * ref.max()
 
 
+@pytest.mark.parametrize("inf_tokens", [1, 70])
+def test_infinities_keep_their_signs(wavec, tuning, inf_tokens):
+    """What infinities and NaNs of the rows give: +inf, -inf, NaN where both signs or a zero weight
+    meet one, as the gathers give (which multiply each row of a segment by its weight)."""
+    rng = np.random.default_rng(inf_tokens)
+    C, cout, K, S, tokens = 400, 112, 3, 72, 70
+    starts = rng.integers(0, C - S + 1, (cout, K))
+    w = synth.normal_f16(rng, (cout, K * S), 0.1)
+    w[rng.random(w.shape) < 0.02] = 0.0
+    w[rng.random(w.shape) < 0.01] = np.float16(-0.0)
+    w[0, 0], w[1, 5] = np.float16(6e-8), np.float16(-6e-8)  # subnormal
+    x = rng.standard_normal((C, 1, tokens)).astype(np.float32)
+    for t in range(inf_tokens):
+        for v in (np.inf, -np.inf, np.nan)[:1 + t % 3]:
+            x[rng.integers(0, C), 0, t] = v
+    got = []
+    for jobs in (1, 0):
+        tuning("jobs", jobs)
+        g = wavec.WaveGraph(kv_cache_max_seq=0)
+        g.add_input("x", C, 1, tokens, is_1d=True)
+        g.add_sparse_wave("w", "x", "y", cluster_rows(starts, S), w, None, cluster=1, act="none")
+        plan = g.compile()
+        got.append(plan.infer_f32(x)[0][:, 0, :])
+        assert plan.exec_report()["waves"][0]["kernel"] == ("jobs" if jobs else "gather_dot")
+        plan.release_gpu()
+    a, b = got
+    assert np.isposinf(b).any() and np.isneginf(b).any() and np.isnan(b).any()
+    for kind in (np.isposinf, np.isneginf, np.isnan):
+        assert np.array_equal(kind(a), kind(b))
+    fin = np.isfinite(b)
+    # two fp16 roundings of fp32 sums of 216 products: half an ulp (2^-11) each, and 2^-20 of the
+    # largest sums between the orders
+    assert np.abs(a[fin] - b[fin]).max() <= 2.0 ** -10 * np.abs(b[fin]).max()
+
+
+def test_infinite_weights_stay_on_the_gathers(wavec, tuning):
+    tuning("jobs", 1)
+    starts = np.arange(64)[:, None] * 4
+    w = np.ones((64, 64), np.float16)
+    for v, kernel in ((1.0, "jobs"), (np.inf, "gather_dot"), (np.nan, "gather_dot")):
+        w[3, 7] = v
+        g = wavec.WaveGraph(kv_cache_max_seq=0)
+        g.add_input("x", 400, 1, 64, is_1d=True)
+        g.add_sparse_wave("w", "x", "y", cluster_rows(starts, 64), w, None, cluster=1)
+        plan = g.compile()
+        plan.init_gpu()
+        assert plan.exec_report()["waves"][0]["kernel"] == kernel
+        plan.release_gpu()
+
+
 @pytest.mark.parametrize("C,cout,K,S,tokens,kernel", [
     (65536, 4096, 8, 64, 64, "jobs"),            # segments overlap 32 times
     (200_000, 512, 8, 128, 64, "jobs"),          # few jobs per window, 11 MiB of fragments
