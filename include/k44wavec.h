@@ -289,7 +289,8 @@ int wavec_gpu_read_canvas_2d(void *handle, unsigned long long elem_off, unsigned
  *   (workgroups x waves) grids where those launch at most 1.5x the work items (automatic);
  *   "embed_refresh" 0 | 1 a decode embedding never / also (automatic) refreshes the compact
  *   state copy of the first layer's folded token shift (0: that RMSNorm + shift runs alone);
- *   "rows" 0 | 1 | 4 | 8 no row-table MFMA kernel / that many waves per tile in it;
+ *   "rows" 0 | 1 | 4 | 8 no row-table MFMA kernel and no offset lists / that many waves per tile
+ *   in it, and lists wherever they apply (1 | 4 waves per neuron; 8: 4);
  *   "jobs" 0 | 1 no MFMA job tiles for private segments / wherever they apply.
  * wavec_set_tuning returns -1 (with a message) for an unknown key or a value the key does not
  * honour: -1 is always accepted; "dma_stages" takes 2 | 4, "ksplit" 1 | 4, "xcd_order" 0..2,

@@ -416,16 +416,37 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
     return true;
 }
 
-// Offset lists of a wave with segments under 32 positions, of 16 and more (the segment gathers'
-// batch) only while the rows of a token tile take at most two XCDs' L2: 4,096 x 8 x 16 of 65,536
-// rows over 256 tokens 33.1 us as segments, 28.7 as lists, 1,024 x 8 x 24 of 20,000 over 64 7.2 and
-// 5.0, but 8,192 x 12 x 16 of 131,072 over 64 20.5 and 25.4.
-// Returns false (nothing set) for those, for rows off the 16-byte grid or beyond 32-bit offsets.
+// Whether offset lists are the faster form of a wave with segments under 32 positions.  A list costs
+// its steps of 32 positions, the segment gathers their batches of 16 positions of one segment, and with
+// few waves both cost their length: the lists' four 128-byte loads against sixteen in flight.  Measured
+// over 48 to 8,192 neurons of 4 and 16 segments of 2 to 31 positions, 64 to 512 tokens, 2.5 to 32 MiB
+// of rows per 64 tokens (the lists' time over the gathers'):
+//  - under 16 gather waves per CU (8 of 256 tokens) 0.30 to 1.07, at the mean 0.73;
+//  - else, over 64- and 128-token slabs, 0.77 where the steps are up to a quarter of the batches (0.39
+//    to 1.09), 0.94 up to two fifths of them while the rows of all tokens fit two XCDs' L2 (0.82 to
+//    1.05), beyond that 1.07, with more steps 1.09 (up to 1.47), but 0.96 with at most two of
+//    them over a 64-token slab;
+//  - over 256-token slabs, whose gathers read 512 bytes of a row at once, 0.83 while a tile's rows
+//    fit two XCDs' L2 (0.52 to 1.13), with under 8 segments below 16 positions 1.09 (0.90 to
+//    1.29); beyond L2 0.85 for steps up to an eighth of the batches, else 1.01 (0.88 to 1.17).
+static bool lists_faster(uint64_t cout, uint32_t K, uint32_t S, uint32_t tokens, uint32_t slab,
+                         uint64_t unique_rows) {
+    const uint64_t l2 = 8ull << 20, steps = (K * S + 31u) / 32u, batches = K * ((S + 15u) / 16u);
+    if (cout * (tokens / slab) < (slab == 256u ? 2048u : 4096u)) return true;
+    if (slab == 256u)
+        return unique_rows * 128u <= l2 ? S >= 16u || K >= 8u : 8u * steps <= batches;
+    return 4u * steps <= batches || (slab == 64u && steps <= 2u) ||
+           (5u * steps <= 2u * batches && unique_rows * tokens * 2u <= l2);
+}
+
+// Offset lists of a wave with segments under 32 positions where they are faster (or "rows" forces
+// them).  Returns false (nothing set) for others, for rows off the 16-byte grid or beyond 32-bit
+// offsets.
 bool K44GpuExecutorState::row_list(const K44ExecCmd &c, WaveExec &wx,
                                    const std::vector<uint16_t> &wraw,
                                    const std::vector<uint64_t> &starts) {
-    if (wx.S >= 32u || (wx.S >= 16u && wx.unique_rows * 128u > (8ull << 20)) ||
-        tune(Tune::Rows) == 0 || wx.tokens % 64u != 0u || wx.step % 8u != 0u ||
+    const int force = tune(Tune::Rows);
+    if (wx.S >= 32u || force == 0 || wx.tokens % 64u != 0u || wx.step % 8u != 0u ||
         wx.out_stride % 8u != 0u || wx.y_off % 8u != 0u || (wx.has_res && wx.res_off % 8u != 0u))
         return false;
     // switches that pick a form of the segment gathers keep them
@@ -437,6 +458,7 @@ bool K44GpuExecutorState::row_list(const K44ExecCmd &c, WaveExec &wx,
     if (hi - lo + (uint64_t)wx.S * wx.step > 0xffffffffull || wx.tokens / 64u > 65535u) return false;
     for (uint64_t s : starts)
         if (s % 8u != 0u) return false;
+    if (force < 0 && !lists_faster(c.Cout, wx.K, wx.S, wx.tokens, wx.slab, wx.unique_rows)) return false;
     const uint32_t fan = wx.K * wx.S, per = (fan + 31u) / 32u * 32u;
     std::vector<uint32_t> ro((size_t)wx.rows * per);
     for (size_t r = 0; r < wx.rows; ++r) {
@@ -457,7 +479,7 @@ bool K44GpuExecutorState::row_list(const K44ExecCmd &c, WaveExec &wx,
     // Four waves per neuron while one would leave the chip at most 2 per CU and each has some steps
     // (256 x 250 over 10 tokens 3.9 us, 5.3 with one; 1,024 x 100 over 64 4.7 and 4.4).
     wx.rl_kw = (uint64_t)c.Cout * (wx.tokens / 64u) <= 512u && per >= 128u ? 4u : 1u;
-    if (tune(Tune::Rows) > 0) wx.rl_kw = tune(Tune::Rows) == 1 ? 1u : 4u;
+    if (force > 0) wx.rl_kw = force == 1 ? 1u : 4u;
     wx.ksplit = wx.rl_kw;
     wx.why += "; lists of row offsets, " + std::to_string(wx.rl_kw) + " waves per neuron";
     return true;

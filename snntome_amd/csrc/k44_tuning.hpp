@@ -57,7 +57,8 @@ enum class Tune : int {
                    //                  where they launch at most 1.5x the work items
     Jobs,          // "jobs":          0 = no MFMA job tiles for private segments, 1 = wherever
                    //                  they apply
-    Rows,          // "rows":          0 = no row-table MFMA kernel, 1 | 4 | 8 = waves per tile in it
+    Rows,          // "rows":          0 = no row-table MFMA kernel and no offset lists, 1 | 4 | 8 =
+                   //                  waves per tile in it, lists wherever they apply (8: 4)
     Count
 };
 

@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
     (16, 1, 1, 1, 1, "none", False), (50, 1, 33, 1, 64, "relu", True),
     (208, 1, 257, 1, 130, "silu", False), (30, 8, 96, 1, 300, "gelu", True),
     (64, 2, 72, 3, 65, "sigmoid", False), (48, 1, 60, 15, 100, "leaky_relu", True),
+    (50, 1, 64, 16, 64, "relu", True), (26, 8, 96, 24, 130, "gelu", False),
+    (37, 1, 310, 31, 256, "silu", False),
 ])
 def test_scattered_private_rows(wavec, orc, tuning, kw, n_rows, cluster, fan, S, tokens, act,
                                 residual):
@@ -56,3 +58,28 @@ def test_infinities_stay_infinite(wavec, tuning):
     y, _ = plan.infer_f32(x)
     assert plan.exec_report()["waves"][0]["kernel"] == "row_list"
     assert np.all(np.isposinf(y[:, 0, ::2])) and np.all(y[:, 0, 1::2] == 0.0)
+
+
+@pytest.mark.parametrize("C,cout,K,S,tokens,kernel", [
+    (131072, 2048, 16, 24, 64, "row_list"),    # few waves
+    (65536, 4096, 16, 24, 64, "row_list"),     # 3/8 of the batches, rows within L2
+    (131072, 4096, 16, 24, 64, "gather_dot"),  # beyond it
+    (20000, 4096, 16, 15, 64, "gather_dot"),   # half of the batches
+    (20000, 4096, 4, 15, 64, "row_list"),      # two steps
+    (131072, 4096, 16, 8, 128, "row_list"),
+    (20000, 4096, 4, 4, 256, "gather_dot"),    # 256-token gathers: few short segments
+    (65536, 4096, 8, 15, 256, "row_list"),
+    (131072, 4096, 8, 15, 256, "gather_dot"),
+    (131072, 4096, 16, 4, 256, "row_list"),
+])
+def test_automatic_choice(wavec, tuning, C, cout, K, S, tokens, kernel):
+    """Each line of the rule from both sides."""
+    rng = np.random.default_rng(S)
+    starts = (rng.integers(0, (C - S) // 8 + 1, (cout, K)) * 8).astype(np.uint32)
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", C, 1, tokens, is_1d=True)
+    g.add_cluster_wave("w", "x", "y", starts, S, np.ones((cout, K * S), np.float16), None, cluster=1)
+    plan = g.compile()
+    plan.init_gpu()
+    assert plan.exec_report()["waves"][0]["kernel"] == kernel
+    plan.release_gpu()
