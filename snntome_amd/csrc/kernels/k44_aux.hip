@@ -280,14 +280,18 @@ __global__ __launch_bounds__(1024) void k44_rmsnorm_regs_kernel(__half *__restri
     }
 }
 
-// Middling token counts (65 .. 8,191): workgroup = 8 tokens x 1,024 channel lanes, each thread's
-// channels in registers from the sum to the store, so the input is read once.  Bound by the
-// gather of 16-byte row pieces: workgroup b works for XCD b % 8 (round-robin dispatch) on a
-// contiguous run of octets, so the 8 octets of a 128-byte line meet in one L2 instead of being
-// fetched by every XCD.  Sums of squares in 64-bit floats (each square is exact in it): 3
-// instructions an element instead of the 25 of the integer limbs that the decode kernels need to
-// be independent of the order.  2,048 tokens x 2,048 channels: 26.8 -> 9.4 us, 200 x
-// 1,024 5.5 -> 4.9.
+// Rows of more than one 64-token tile that the kernel above does not take (fewer than 8,192 tokens,
+// a count that is no multiple of 32, or more than 4,096 channels): workgroup = 8 tokens x 1,024
+// channel lanes, each thread's channels in registers from the sum to the store, so the input is
+// read once.  Bound by the gather of 16-byte row pieces: workgroup b works for XCD b % 8
+// (round-robin dispatch) on a contiguous run of octets, so the 8 octets of a 128-byte line meet
+// in one L2 instead of being fetched by every XCD.
+// The sum of squares is the exact one rounded to fp32 once, as that of the integer limbs
+// (k44_sumsq.hpp), whatever the order: squares (exact) are added in 64-bit floats, at most 30
+// roundings of 2^-53 on the way, and where fp32 could round the exact sum either way (one token in
+// 2^23 of ordinary data) the workgroup adds its registers again without rounding.
+// 3 instructions an element instead of 25: 2,048 tokens x 2,048 channels 26.7 -> 9.6 us, 200 x
+// 1,024 5.4 -> 5.1 (with the exact sums for every token: 10.6 and 5.9).
 __device__ __forceinline__ double shfl_xor_f64(double v, int m) {
     const uint64_t b = __builtin_bit_cast(uint64_t, v);
     const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)b, m, 64);
@@ -295,13 +299,40 @@ __device__ __forceinline__ double shfl_xor_f64(double v, int m) {
     return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
 }
 
+// Sums over a wave of 8 tokens' values per lane.  At each of the first three steps a lane hands over
+// half of its tokens, so lane l ends with token 4 (l & 1) + 2 (l >> 1 & 1) + (l >> 2 & 1) summed over 8
+// lanes; then plain.  Lanes 0..7 store their tokens' sums.
+__device__ __forceinline__ void octet_wave_sums(double (&s)[8], uint32_t lane, double *out) {
+#pragma unroll
+    for (int m = 1, w = 4; m < 8; m <<= 1, w >>= 1) {
+        const bool up = (lane & (uint32_t)m) != 0u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k >= w) continue;
+            const double keep = up ? s[k + w] : s[k], give = up ? s[k] : s[k + w];
+            s[k] = keep + shfl_xor_f64(give, m);
+        }
+    }
+#pragma unroll
+    for (int m = 8; m < 64; m <<= 1) s[0] += shfl_xor_f64(s[0], m);
+    if (lane < 8u) out[4u * (lane & 1u) + (lane & 2u) + (lane >> 2)] = s[0];
+}
+
+// a + b (both >= 0) rounded to fp32 once, nearest even: rounded to odd at 53 bits first.
+__device__ __forceinline__ float sum2_f32(double a, double b) {
+    const double s = a + b, bb = s - a, e = (a - (s - bb)) + (b - bb);
+    uint64_t u = __builtin_bit_cast(uint64_t, s);
+    if (e != 0.0 && (u & 1u) == 0u) u += e > 0.0 ? 1u : ~0ull;
+    return (float)__builtin_bit_cast(double, u);
+}
+
 template <int CPT>
-__global__ __launch_bounds__(1024) void k44_rmsnorm_octet_kernel(__half *__restrict__ y,
+__global__ __launch_bounds__(1024, CPT <= 2 ? 8 : 4) void k44_rmsnorm_octet_kernel(__half *__restrict__ y,
                                                                  const __half *__restrict__ x,
                                                                  const __half *__restrict__ gamma,
                                                                  uint32_t D, uint32_t stride,
                                                                  float eps) {
-    __shared__ double part[16][8];
+    __shared__ double part[16][8], rest[16][8];
     __shared__ float inv_s[8];
     const uint32_t n = gridDim.x, xcd = blockIdx.x & 7u, q = n >> 3, r = n & 7u;
     const uint32_t t0 = (xcd * q + min(xcd, r) + (blockIdx.x >> 3)) * 8u;
@@ -326,29 +357,65 @@ __global__ __launch_bounds__(1024) void k44_rmsnorm_octet_kernel(__half *__restr
             ss[k] = fma(f, f, ss[k]);
         }
     }
-    // Wave sums: at each of the first three steps a lane hands over half of its tokens, so lane l
-    // ends with token 4 (l & 1) + 2 (l >> 1 & 1) + (l >> 2 & 1) summed over 8 lanes; then plain.
-#pragma unroll
-    for (int m = 1, w = 4; m < 8; m <<= 1, w >>= 1) {
-        const bool up = (lane & (uint32_t)m) != 0u;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (k >= w) continue;
-            const double keep = up ? ss[k + w] : ss[k], give = up ? ss[k] : ss[k + w];
-            ss[k] = keep + shfl_xor_f64(give, m);
-        }
-    }
-#pragma unroll
-    for (int m = 8; m < 64; m <<= 1) ss[0] += shfl_xor_f64(ss[0], m);
-    if (lane < 8u) part[wave][4u * (lane & 1u) + (lane & 2u) + (lane >> 2)] = ss[0];
+    octet_wave_sums(ss, lane, part[wave]);
     __syncthreads();
     if (tid < 8u) {
         double t = part[0][tid];
 #pragma unroll
         for (int w = 1; w < 16; ++w) t += part[w][tid];
-        inv_s[tid] = rsqrtf((float)t / (float)D + eps);
+        const float f = (float)(t - t * 0x1p-48);
+        // (an infinite or NaN sum is one in any order; -1: not decided)
+        inv_s[tid] = t != t ? __builtin_nanf("")
+                     : f == (float)(t + t * 0x1p-48) || t > 0x1p60 ? rsqrtf((float)t / (float)D + eps)
+                                                                   : -1.0f;
     }
     __syncthreads();
+    bool again = false;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) again = again || inv_s[k] == -1.0f;
+    // the fp16 values are what stays in registers, not their conversions
+    auto opaque = [&] {
+#pragma unroll
+        for (int u = 0; u < CPT; ++u) asm volatile("" : "+v"(v[u].x), "+v"(v[u].y), "+v"(v[u].z), "+v"(v[u].w));
+    };
+    opaque();
+    if (again) {  // (the whole workgroup)
+        // A square is a multiple of 2^-48 below 2^32: the multiples of 2^-8 (hi, < 2^45 over 8,192
+        // channels) and what they leave (lo, < 2^4) each fit 53 bits.  2^44 + hi has the unit 2^-8.
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            __builtin_amdgcn_sched_barrier(0);  // (a token at a time: or the registers spill)
+            double hi = 0x1p44, lo = 0.0;
+#pragma unroll
+            for (int u = 0; u < CPT; ++u) {
+                const double f = (double)__half2float(reinterpret_cast<const __half *>(&v[u])[k]);
+                const double q = f * f, t = hi + q;
+                lo += q - (t - hi);
+                hi = t;
+            }
+            hi -= 0x1p44;
+#pragma unroll
+            for (int m = 1; m < 64; m <<= 1) {
+                hi += shfl_xor_f64(hi, m);
+                lo += shfl_xor_f64(lo, m);
+            }
+            if (lane == 0u) {
+                part[wave][k] = hi;
+                rest[wave][k] = lo;
+            }
+        }
+        __syncthreads();
+        if (tid < 8u && inv_s[tid] == -1.0f) {
+            double a = part[0][tid], b = rest[0][tid];
+            for (int w = 1; w < 16; ++w) {
+                a += part[w][tid];
+                b += rest[w][tid];
+            }
+            inv_s[tid] = rsqrtf(sum2_f32(a, b) / (float)D + eps);
+        }
+        __syncthreads();
+        opaque();
+    }
     float inv[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) inv[k] = inv_s[k];

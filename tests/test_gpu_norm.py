@@ -1,5 +1,8 @@
-"""RMSNorm over 65 to 8,191 tokens (one octet of tokens per workgroup, sums in 64-bit floats) at the
-edges of its channels per thread and token octets, against a float64 norm of the fp16 input."""
+"""RMSNorm over rows of more than one 64-token tile (one octet of tokens per workgroup) at the edges of
+its channels per thread and token octets, against a float64 norm of the fp16 input; its sums of
+squares are exact, bit for bit the scales of the kernel for up to 64 tokens."""
+import math
+
 import numpy as np
 import pytest
 
@@ -15,7 +18,8 @@ def _plan(wavec, D, T, gamma):
 
 
 @pytest.mark.parametrize("D,T", [(1024, 65), (1025, 100), (2048, 2048), (3000, 777), (4097, 130),
-                                 (8192, 72), (8193, 70), (768, 200), (767, 200), (2048, 8190)])
+                                 (8192, 72), (8193, 70), (768, 200), (767, 200), (2048, 8190),
+                                 (768, 8200), (5000, 8224)])
 def test_middling_token_counts(wavec, D, T):
     rng = np.random.default_rng(D + T)
     gamma = (1.0 + 0.1 * rng.standard_normal(D)).astype(np.float32)
@@ -45,3 +49,36 @@ def test_infinities_and_nans(wavec):
     assert np.all(np.isnan(y[:, 0, 12]))
     rest = np.delete(y[:, 0, :], [3, 12], axis=1)
     assert np.all(np.abs(rest - 1.0) < 2e-3)
+
+
+def _tie_token(rng, D):
+    """D fp16 values whose sum of squares lies 2^-48 beside the middle of two fp32 values."""
+    x = rng.permutation(np.concatenate([rng.standard_normal(D - 64), np.zeros(64)])).astype(np.float16)
+    units = lambda v: int(round(float(v) * 2.0 ** 24))  # exact: fp16 values are multiples of 2^-24
+    free = list(np.flatnonzero(x == 0))
+    total = sum(units(v) ** 2 for v in x)
+    ulp = 1 << (total.bit_length() - 24)
+    target = total // ulp * ulp + ulp // 2 + ulp + int(rng.choice([-1, 1]))
+    while total < target:  # the rest as squares, largest first (11-bit significands)
+        m = math.isqrt(target - total)
+        drop = max(0, m.bit_length() - 11)
+        m = m >> drop << drop
+        x[free.pop()] = np.float16(m * 2.0 ** -24)
+        total += m * m
+    assert sum(units(v) ** 2 for v in x) == target and target.bit_length() - 24 == ulp.bit_length() - 1
+    return x
+
+
+@pytest.mark.parametrize("D", [768, 2048, 4096, 8192])
+def test_sums_are_exact(wavec, D):
+    """Sums next to the middle of two fp32 values, where a sum rounded on the way gives the other
+    one: the outputs are those of the exact integer sums that run up to 64 tokens."""
+    rng = np.random.default_rng(D)
+    T = 640
+    x = np.stack([_tie_token(rng, D) for _ in range(T)], 1)
+    gamma = (1.0 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    y, _ = _plan(wavec, D, T, gamma).infer_f32(x.astype(np.float32)[:, None, :])
+    few = _plan(wavec, D, 64, gamma)
+    for t in range(0, T, 64):
+        want, _ = few.infer_f32(x[:, t:t + 64].astype(np.float32)[:, None, :])
+        assert np.array_equal(y[:, 0, t:t + 64].view(np.uint32), want[:, 0].view(np.uint32)), t
