@@ -204,7 +204,7 @@ void K44GpuExecutorState::launch_group(const MfmaGroupExec &g) {
     if (g.rowsk) {
         const WaveExec &w = *waves[g.members[0]];
         k44dev::RowsLaunch l;
-            if (g.members.size() > 1u) {
+        if (g.members.size() > 1u) {
             l.waves = g.rk_args.p;
             l.start = g.start.p;
             l.n = (uint32_t)g.members.size();
@@ -397,50 +397,69 @@ void K44GpuExecutorState::upload_input_f32(const float *in, size_t n) {
     }
 }
 
-// Device address of [p, p + bytes) if all of it is one page-locked host allocation, else null.
-static void *page_locked(void *p, size_t bytes) {
+// How a read reaches [p, p + bytes): in place at `direct` if all of it is one page-locked host
+// allocation or memory of the executor's GPU; else through the ring, by the runtime's copy to memory
+// of another GPU (`device`), by the host to its own.
+struct Target {
+    void *direct;
+    bool device;
+};
+static Target target_of(void *p, size_t bytes) {
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        return {nullptr, false};
     }
-    if (at.type != hipMemoryTypeHost || !at.devicePointer) return nullptr;
+    const bool device = at.type == hipMemoryTypeDevice;
+    int gpu = 0;
+    K44_HIP(hipGetDevice(&gpu));
+    if ((!device && at.type != hipMemoryTypeHost) || (device && at.device != gpu) ||
+        !at.devicePointer)
+        return {nullptr, device};
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
     if (hipMemGetAddressRange(&base, &size, reinterpret_cast<hipDeviceptr_t>(at.devicePointer)) !=
         hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        return {nullptr, device};
     }
     const size_t skip = static_cast<char *>(at.devicePointer) - static_cast<char *>(base);
-    return skip <= size && bytes <= size - skip ? at.devicePointer : nullptr;
+    return {skip <= size && bytes <= size - skip ? at.devicePointer : nullptr, device};
 }
 
-// Fills host memory from a kernel and waits for it: fill(target, first byte, bytes) enqueues a
-// kernel that writes that part of the output to `target`.  Page-locked destinations are written
-// in place, without a staging buffer and the copy after it (0.5 MB of a 64-token wave: 43 -> 33 us
-// around the plan's run); others through the ring, one chunk copied out while a kernel writes the
-// next (a copy to pageable memory of 4 MB takes 234 us, the ring 110).
+// Fills caller memory from a kernel and waits for it: fill(target, first byte, bytes) enqueues a
+// kernel that writes that part of the output to `target`.  Page-locked
+// destinations are written in place, without a staging buffer and the copy after it (0.5 MB of a
+// 64-token wave: 43 -> 33 us around the plan's run); others through the ring, one chunk copied out
+// while a kernel writes the next (a copy to pageable memory of 4 MB takes 250 us, the ring 187; of
+// 1 GB 64 ms, 44).
 template <typename Fill>
 void K44GpuExecutorState::to_host(void *dst, size_t bytes, Fill &&fill) {
-    if (void *direct = page_locked(dst, bytes)) {
-        fill(direct, 0u, bytes);
+    const Target to = target_of(dst, bytes);
+    if (to.direct) {
+        fill(to.direct, 0u, bytes);
         K44_HIP(hipStreamSynchronize(stream));
         return;
     }
     std::lock_guard<std::recursive_mutex> lk(io);
     constexpr size_t kChunk = HostRing::kChunk;
+    auto out = [&](size_t at, const char *from, size_t n) {
+        char *d = static_cast<char *>(dst) + at;
+        if (to.device)
+            K44_HIP(hipMemcpy(d, from, n, hipMemcpyDefault));
+        else
+            std::memcpy(d, from, n);
+    };
     if (bytes <= kChunk) {
         fill(ring.p, 0u, bytes);
         K44_HIP(hipStreamSynchronize(stream));
-        std::memcpy(dst, ring.p, bytes);
+        out(0u, ring.p, bytes);
         return;
     }
     const size_t chunks = (bytes + kChunk - 1u) / kChunk;
     auto take = [&](size_t i) {
         K44_HIP(hipEventSynchronize(ring.ev[i & 1u]));
-        std::memcpy(static_cast<char *>(dst) + i * kChunk, ring.p + (i & 1u) * kChunk,
-                    std::min(kChunk, bytes - i * kChunk));
+        out(i * kChunk, ring.p + (i & 1u) * kChunk, std::min(kChunk, bytes - i * kChunk));
     };
     for (size_t i = 0; i < chunks; ++i) {
         if (i >= 2u) take(i - 2u);

@@ -155,3 +155,47 @@ def test_canvas_reads(wavec, pinned, shift, rows, stride, cols, off):
     finally:
         del buf
         hip.hipHostFree(p)
+
+
+def _read_2d(plan, addr, off, rows, stride, cols):
+    assert plan._lib.wavec_gpu_read_canvas_2d(plan._handle, off, rows, stride, cols,
+                                              ctypes.cast(addr, ctypes.POINTER(ctypes.c_uint16))) == 0
+
+
+def _filled_plan(wavec, channels=2100):
+    """A plan whose first rows hold known words: (plan, words [channels * 1024])."""
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", channels, 1, 1024, is_1d=True)
+    g.add_swiglu("m", "x", "x", "y")
+    plan = g.compile()
+    plan.init_gpu()
+    data = np.random.default_rng(channels).integers(0, 65536, channels * 1024, dtype=np.uint16)
+    plan.write_canvas(0, data)
+    return plan, data
+
+
+@pytest.mark.parametrize("rows,stride,cols,shift", [(1, 5, 5, 0), (40, 64, 64, 8), (900, 1024, 1000, 1)])
+def test_reads_into_device_memory(wavec, rows, stride, cols, shift):
+    """A destination on the GPU (as a copy takes it), up to several transfer chunks."""
+    plan, data = _filled_plan(wavec)
+    want = np.lib.stride_tricks.as_strided(data, (rows, cols), (2 * stride, 2)).reshape(-1)
+    n = shift + want.size + 8
+    hip, d = _hip(), ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(d), ctypes.c_size_t(2 * n)) == 0
+    try:
+        for two_d in (True, False):
+            got = np.full(n, 0x5a5a, np.uint16)
+            size, mem = ctypes.c_size_t(2 * n), got.ctypes.data_as(ctypes.c_void_p)
+            assert hip.hipMemcpy(d, mem, size, 1) == 0  # host to device
+            if two_d:
+                _read_2d(plan, d.value + 2 * shift, 0, rows, stride, cols)
+            else:
+                want = data[:want.size]
+                assert plan._lib.wavec_gpu_read_canvas(
+                    plan._handle, 0, want.size,
+                    ctypes.cast(d.value + 2 * shift, ctypes.POINTER(ctypes.c_uint16))) == 0
+            assert hip.hipMemcpy(mem, d, size, 2) == 0  # device to host
+            assert np.array_equal(got[shift:shift + want.size], want)
+            assert np.all(got[:shift] == 0x5a5a) and np.all(got[shift + want.size:] == 0x5a5a)
+    finally:
+        hip.hipFree(d)
