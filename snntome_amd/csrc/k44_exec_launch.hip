@@ -398,13 +398,13 @@ void K44GpuExecutorState::upload_input_f32(const float *in, size_t n) {
 }
 
 // How a read reaches [p, p + bytes): in place at `direct` if all of it is one page-locked host
-// allocation or memory of the executor's GPU; else through the ring, by the runtime's copy to memory
-// of another GPU (`device`), by the host to its own.
+// allocation or memory of the executor's GPU, aligned as the kernels store; else through the ring,
+// by the runtime's copy to memory of another GPU (`device`), by the host to its own.
 struct Target {
     void *direct;
     bool device;
 };
-static Target target_of(void *p, size_t bytes) {
+static Target target_of(void *p, size_t bytes, size_t align) {
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();
@@ -414,7 +414,7 @@ static Target target_of(void *p, size_t bytes) {
     int gpu = 0;
     K44_HIP(hipGetDevice(&gpu));
     if ((!device && at.type != hipMemoryTypeHost) || (device && at.device != gpu) ||
-        !at.devicePointer)
+        !at.devicePointer || reinterpret_cast<uintptr_t>(at.devicePointer) % align != 0u)
         return {nullptr, device};
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
@@ -428,14 +428,14 @@ static Target target_of(void *p, size_t bytes) {
 }
 
 // Fills caller memory from a kernel and waits for it: fill(target, first byte, bytes) enqueues a
-// kernel that writes that part of the output to `target`.  Page-locked
+// kernel that writes that part of the output to `target`, `align` bytes a value.  Page-locked
 // destinations are written in place, without a staging buffer and the copy after it (0.5 MB of a
 // 64-token wave: 43 -> 33 us around the plan's run); others through the ring, one chunk copied out
 // while a kernel writes the next (a copy to pageable memory of 4 MB takes 250 us, the ring 187; of
 // 1 GB 64 ms, 44).
 template <typename Fill>
-void K44GpuExecutorState::to_host(void *dst, size_t bytes, Fill &&fill) {
-    const Target to = target_of(dst, bytes);
+void K44GpuExecutorState::to_host(void *dst, size_t bytes, size_t align, Fill &&fill) {
+    const Target to = target_of(dst, bytes, align);
     if (to.direct) {
         fill(to.direct, 0u, bytes);
         K44_HIP(hipStreamSynchronize(stream));
@@ -474,7 +474,7 @@ void K44GpuExecutorState::download_output_f32(float *out, size_t n) {
     const k44dev::FrameLayout f = frame_layout(layout(plan_meta.output_res_key),
                                                 plan_meta.output_h, plan_meta.output_w);
     const uint16_t *region = reinterpret_cast<const uint16_t *>(canvas.p + plan_meta.output_off);
-    to_host(out, n * 4u, [&](void *to, size_t first, size_t bytes) {
+    to_host(out, n * 4u, 4u, [&](void *to, size_t first, size_t bytes) {
         K44_HIP(k44dev::launch_export_f32(static_cast<float *>(to), region, first / 4u, bytes / 4u,
                                           f, stream));
     });
@@ -483,7 +483,7 @@ void K44GpuExecutorState::download_output_f32(float *out, size_t n) {
 void K44GpuExecutorState::read_rows(uint16_t *dst, uint64_t off, uint64_t rows, uint64_t row_stride,
                                     uint64_t cols) {
     const uint16_t *src = reinterpret_cast<const uint16_t *>(canvas.p + off);
-    to_host(dst, rows * cols * 2u, [&](void *to, size_t first, size_t bytes) {
+    to_host(dst, rows * cols * 2u, 2u, [&](void *to, size_t first, size_t bytes) {
         K44_HIP(k44dev::launch_pack_rows(static_cast<uint16_t *>(to), src, first / 2u, bytes / 2u,
                                          row_stride, cols, stream));
     });

@@ -465,7 +465,7 @@ struct K44GpuExecutorState {
     void download_output_f32(float *out, size_t n);
     void read_rows(uint16_t *dst, uint64_t off, uint64_t rows, uint64_t row_stride, uint64_t cols);
     template <typename Fill>
-    void to_host(void *dst, size_t bytes, Fill &&fill);
+    void to_host(void *dst, size_t bytes, size_t align, Fill &&fill);
     int infer_f32(const float *in, int in_elems, float *out, int out_elems, float *ms_out);
 };
 

@@ -1,6 +1,7 @@
 """infer_f32's device conversions: the canvas region it writes and the floats it returns, bit for
 bit against the host rounding rules, on every layout and at the values where rounding can go
 wrong (ties, subnormals, overflow, NaN payloads)."""
+import contextlib
 import ctypes
 
 import numpy as np
@@ -199,3 +200,26 @@ def test_reads_into_device_memory(wavec, rows, stride, cols, shift):
             assert np.all(got[:shift] == 0x5a5a) and np.all(got[shift + want.size:] == 0x5a5a)
     finally:
         hip.hipFree(d)
+
+
+@contextlib.contextmanager
+def _page_locked(n_bytes):
+    hip, p = _hip(), ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(n_bytes), 0) == 0
+    try:
+        yield p.value
+    finally:
+        hip.hipHostFree(p)
+
+
+def test_page_locked_reads_off_the_element_grid(wavec):
+    """Destinations at odd bytes of page-locked memory (a host copy does not mind them)."""
+    plan, data = _filled_plan(wavec, 700)
+    with _page_locked(1 << 20) as base:
+        mem = np.ctypeslib.as_array(ctypes.cast(base, ctypes.POINTER(ctypes.c_uint8)), (1 << 20,))
+        for odd, rows, cols in ((1, 3, 5), (7, 64, 1024), (3, 300, 640)):
+            mem[:] = 0xab
+            _read_2d(plan, base + odd, 0, rows, 1024, cols)
+            want = np.ascontiguousarray(data.reshape(-1, 1024)[:rows, :cols]).view(np.uint8).ravel()
+            assert np.array_equal(mem[odd:odd + want.size], want)
+            assert np.all(mem[:odd] == 0xab) and np.all(mem[odd + want.size:] == 0xab)
