@@ -3,6 +3,7 @@ bit against the host rounding rules, on every layout and at the values where rou
 wrong (ties, subnormals, overflow, NaN payloads)."""
 import contextlib
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -223,3 +224,71 @@ def test_page_locked_reads_off_the_element_grid(wavec):
             want = np.ascontiguousarray(data.reshape(-1, 1024)[:rows, :cols]).view(np.uint8).ravel()
             assert np.array_equal(mem[odd:odd + want.size], want)
             assert np.all(mem[:odd] == 0xab) and np.all(mem[odd + want.size:] == 0xab)
+
+
+@pytest.mark.parametrize("byte", [0, 4, 2])
+@pytest.mark.parametrize("C,W", [(5, 200), (1500, 1024)])
+def test_infer_into_page_locked_memory(wavec, C, W, byte):
+    """Results written in place, on the 16-byte grid, off it, and off the element grid."""
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", C, 1, W, is_1d=True)
+    g.add_swiglu("m", "x", "x", "y")
+    g.set_output("y")
+    plan = g.compile()
+    x = np.random.default_rng(W).standard_normal((C, 1, W)).astype(np.float32)
+    want = plan.infer_f32(x)[0]
+    fp = ctypes.POINTER(ctypes.c_float)
+    with _page_locked(want.nbytes + 64) as base:
+        mem = np.ctypeslib.as_array(ctypes.cast(base, ctypes.POINTER(ctypes.c_uint8)), (want.nbytes + 64,))
+        mem[:] = 0xab
+        assert plan._lib.wavec_gpu_infer_f32(plan._handle, x.ctypes.data_as(fp), x.size,
+                                             ctypes.cast(base + byte, fp), want.size, None) == 0
+        assert np.array_equal(mem[byte:byte + want.nbytes], want.view(np.uint8).ravel())
+        assert np.all(mem[:byte] == 0xab) and np.all(mem[byte + want.nbytes:] == 0xab)
+
+
+@pytest.mark.parametrize("C,W,extra", [(37, 200_000, 0), (5, 5_000_000, 0), (37, 200_000, 2_500_001)])
+def test_inputs_of_several_stages(wavec, C, W, extra):
+    """Inputs beyond the 16 MiB stage: several channels a pass, one channel larger than it, and one
+    that ends inside a pass."""
+    rng = np.random.default_rng(C)
+    g = wavec.WaveGraph(kv_cache_max_seq=0)
+    g.add_input("x", C, 1, W, is_1d=True)
+    g.add_sparse_wave("w", "x", "y", np.zeros((16, 4), np.uint32), np.ones((16, 4), np.float16), None,
+                      cluster=1)
+    g.set_output("y")
+    plan = g.compile()
+    plan.init_gpu()
+    stride = (W + 63) // 64 * 64
+    off = int(plan.cmds[0]["src_off"])
+    plan.write_canvas(off, np.full(C * stride, 7.0, np.float16))
+    n = C * W - extra
+    x = rng.standard_normal(n, dtype=np.float32)
+    y = np.zeros(1, np.float32)
+    fp = ctypes.POINTER(ctypes.c_float)
+    assert plan._lib.wavec_gpu_infer_f32(plan._handle, x.ctypes.data_as(fp), n, y.ctypes.data_as(fp), 1,
+                                         None) == 0
+    want = np.zeros((C, stride), np.float16)
+    full = np.zeros(C * W, np.float16)
+    full[:n] = x.astype(np.float16)
+    want[:, :W] = full.reshape(C, W)
+    assert np.array_equal(plan.read_canvas(off, C * stride), want.view(np.uint16).ravel())
+
+
+def test_threads_reading_one_plan(wavec):
+    """Threads that read different rows of one plan into pageable memory share its transfer ring."""
+    plan, data = _filled_plan(wavec)
+    jobs = [(0, 2048), (1024 * 100, 1 << 20), (1024 * 1000, 700_001), (7, 64)]
+    wrong = []
+
+    def work(off, n):
+        for _ in range(20):
+            if not np.array_equal(plan.read_canvas(off, n), data[off:off + n]):
+                wrong.append((off, n))
+
+    ts = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong
