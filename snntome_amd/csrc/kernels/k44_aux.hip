@@ -1096,9 +1096,9 @@ hipError_t launch_rmsnorm(__half *y, const __half *x, const __half *gamma, uint3
 #undef K44_RMSW
         return hipGetLastError();
     }
-    // Rows of more than one 64-token tile (decode norms, whose exact sums meet those of folded
-    // producers, keep the kernel below), channels within 8 per thread; below 768 channels most of
-    // the 1,024 lanes idle (512 x 4,096 tokens 7.7 us below, 8.3 here; 768: 11.6 and 9.1).
+    // Rows of more than one 64-token tile (one tile gives too few octets: the kernel below splits its
+    // channels over workgroups), channels within 8 per thread; below 768 channels most of the 1,024
+    // lanes idle (512 x 4,096 tokens 7.5 us below, 8.2 here; 768: 11.5 and 8.9).
     if (!shift && !slots && stride > 64u && D >= 768u && D <= 8u * 1024u) {
         const uint32_t cpt = (D + 1023u) / 1024u;
 #define K44_RMSO(C)                                                                              \

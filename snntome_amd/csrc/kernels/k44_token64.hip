@@ -12,10 +12,10 @@
 // the widest that divides the cluster); a workgroup holds 4 waves on 4 consecutive tiles (same
 // neurons, so the A fragments are shared through L1), or, while such tiles are too few to fill
 // the GPU, KW waves on one tile that share its k-steps (k = wave, wave + KW, ...) and add their
-// sums in LDS in a fixed order: one tile x 2,048 neurons of 512 inputs 16.1 -> 6.2 us, 5 tiles
-// x 4,080 neurons in clusters of 48 (three blocks a wave instead of one) 22.9 -> 13.1 us.  Per 32-deep k-step the wave gathers its
-// 32 index rows (128 bytes each, 8 lanes x 16 bytes per row) into a private LDS tile, and the B
-// operand of v_mfma_f32_16x16x32_f16 comes out with ds_read_b64_tr_b16 (8 positions of one
+// sums in LDS in a fixed order: one tile x 2,048 neurons of 512 inputs 16.0 -> 6.1 us, 5 tiles
+// x 4,080 neurons in clusters of 48 (three blocks a wave instead of one) 22.7 -> 12.6 us.  Per
+// 32-deep k-step the wave gathers its 32 index rows (128 bytes each, 8 lanes x 16 bytes per row)
+// into a private LDS tile, and the B operand of v_mfma_f32_16x16x32_f16 comes out with ds_read_b64_tr_b16 (8 positions of one
 // token per lane), exactly as in the dense-cluster tile kernel.  A fragments are read straight
 // from the WMMA-ordered weights: MFMA lane l needs row 16*nb + (l & 15), columns 32*ks + 8*(l>>4)
 // .. +8, which is WMMA vector ((nb * B_vec16 + 2*ks + (l >> 5)) * 32 + (l & 31)).  The next
