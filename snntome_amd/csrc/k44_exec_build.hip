@@ -355,14 +355,14 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
         best = steps;
         wx.jb_ksteps = ks;
     }
-    // Fragments, zero-padded to 32 jobs per window: at most 3 times the weights, or 32 MiB (all
-    // L2s) where jobs are too far apart for that.  Beyond, memory and set-up grow without bound (a
-    // job per tile holds 32 times its weights) and the time goes with them: 4,096 x 16 x 128 over
-    // 64 tokens of 4 M positions 390 MB of fragments, 179 us, 145 gathered; 4,096 x 8 x 64 of 1 M
-    // 86 MB, 40 and 40; 2,048 x 4 x 256 over 128 tokens of 1 M 109 MB, 74 and 75.  (Some would still
-    // gain, as 4,096 x 16 x 512 over 64 tokens of 1 M positions: 172 and 513 for 7 times the weights.)
+    // Fragments, zero-padded to 32 jobs per window: at most 8 times the weights, twice the rows read
+    // or 32 MiB (all L2s).  Beyond, jobs are too far apart for tiles, whose memory and set-up grow to
+    // 32 times the weights: 4,096 x 16 x 512 over 64 tokens of 8 M positions 1.6 GB, 590 us, 662
+    // gathered; of 2 M 773 MB for 67 MB (281 and 547, given up for the memory); of 1 M 457 MB, 172
+    // and 513, within it.
     const uint64_t frag = best * k44dev::K44_JOB_BLOCKS * 1024u;
-    if (frag > std::max<uint64_t>(32ull << 20, 3u * n_jobs * wx.S * 2u)) return false;
+    const uint64_t row_bytes = wx.unique_rows * wx.tokens * 2u;
+    if (frag > std::max({(uint64_t)(32ull << 20), 8u * n_jobs * wx.S * 2u, 2u * row_bytes})) return false;
     // Times in us that fit both forms over 96 to 8,192 neurons of 2 to 16 segments of 32 to 512
     // positions over 16 to 256 tokens.  Job tiles: 0.35 ns per tile's k-step and 64 tokens, the
     // sums at 5 TB/s, the chain of gathers.  The VALU gathers: their bytes at 22 TB/s from L2, 9
@@ -374,10 +374,16 @@ bool K44GpuExecutorState::job_tiles(const K44ExecCmd &c, WaveExec &wx,
     double t_jobs = 6.0 + 0.25 * wx.jb_ksteps + 0.00035 * (double)best * t64 + 1.6 * mb;
     double t_valu = std::max(2.0 + 0.0135 * wx.K * wx.S,
                              4.0 + 2.0 * mb * wx.S / (x_mb <= 32.0 ? 22.0 : 9.0));
-    // Beyond the 256 MB MALL everything that a form reads once comes from HBM, at 6.5 TB/s.
-    const double rows_mb = (double)wx.unique_rows * wx.tokens * 2e-6, all_mb = rows_mb + (double)frag * 1e-6;
-    if (all_mb > 256.0) t_jobs = std::max(t_jobs, all_mb / 6.5);
-    if (rows_mb > 256.0) t_valu = std::max(t_valu, rows_mb / 6.5);
+    // Rows and fragments beyond the L2s: job tiles take them at 4.7 TB/s (4,096 x 16 x 128 over 64
+    // tokens of 4 M positions 850 MB, 179 us, 145 gathered; 4,096 x 8 x 64 of 1 M 203 MB, 40 and
+    // 40; 2,048 x 4 x 256 over 128 tokens of 1 M 341 MB, 74 and 75; but 4,096 x 8 x 128 over 256
+    // of 512 k 344 MB, 97 and 285), a gathering neuron's chain twice as long (512 x 8 x 128 over 64
+    // of 1 M 21 and 30).
+    const double all_mb = (double)(row_bytes + frag) * 1e-6;
+    if (all_mb > 32.0) {
+        t_jobs = std::max(t_jobs, 6.0 + all_mb / 4.7);
+        t_valu = std::max({t_valu, 2.0 + 0.027 * wx.K * wx.S, (double)row_bytes * 1e-6 / 6.5});
+    }
     if (force < 0 && t_jobs >= 0.85 * t_valu) return false;
     std::vector<uint32_t> first;
     wx.jb_tiles = (uint32_t)cut(wx.jb_ksteps, &first);

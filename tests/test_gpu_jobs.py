@@ -122,11 +122,14 @@ def test_infinite_weights_stay_on_the_gathers(wavec, tuning):
 @pytest.mark.parametrize("C,cout,K,S,tokens,kernel", [
     (65536, 4096, 8, 64, 64, "jobs"),            # segments overlap 32 times
     (200_000, 512, 8, 128, 64, "jobs"),          # few jobs per window, 11 MiB of fragments
-    (1 << 20, 2048, 4, 256, 128, "gather_dot"),  # 109 MB of fragments for 4 MB of weights
-    (1 << 20, 4096, 8, 64, 64, "gather_dot"),    # 86 MB for 4
+    (1 << 18, 2048, 4, 256, 128, "jobs"),        # 54 MB of fragments for 4 MB of weights, 67 MB of rows
+    (1 << 20, 2048, 4, 256, 128, "gather_dot"),  # 109 MB: their traffic outweighs the overlap
+    (1 << 20, 4096, 8, 64, 64, "gather_dot"),    # 86 MB
+    (1 << 19, 2048, 8, 512, 64, "gather_dot"),   # 210 MB for 17 of weights and 67 of rows: too much memory
 ])
 def test_automatic_choice(wavec, tuning, C, cout, K, S, tokens, kernel):
-    """Job tiles where segments overlap; not where their padded fragments would grow without bound."""
+    """Job tiles where segments overlap; not where their padded fragments would
+    grow without bound or cost more than the gathers."""
     rng = np.random.default_rng(S)
     starts = (rng.integers(0, (C - S) // 8 + 1, (cout, K)) * 8).astype(np.uint32)
     g = wavec.WaveGraph(kv_cache_max_seq=0)
