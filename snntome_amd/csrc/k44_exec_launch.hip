@@ -411,9 +411,9 @@ static Target target_of(void *p, size_t bytes, size_t align) {
         return {nullptr, false};
     }
     const bool device = at.type == hipMemoryTypeDevice;
-    int gpu = 0;
-    K44_HIP(hipGetDevice(&gpu));
-    if ((!device && at.type != hipMemoryTypeHost) || (device && at.device != gpu) ||
+    int gpu = at.device;
+    if (device) K44_HIP(hipGetDevice(&gpu));
+    if ((!device && at.type != hipMemoryTypeHost) || at.device != gpu ||
         !at.devicePointer || reinterpret_cast<uintptr_t>(at.devicePointer) % align != 0u)
         return {nullptr, device};
     hipDeviceptr_t base = nullptr;
